@@ -836,6 +836,10 @@ size_t nsmlp_prefill_workspace_bytes(int H, int NB, int M, int k) {
   } else {
     off += align_up(nk * 32 * 2);                  // act per (block, token) entry
   }
+  if (few_tokens_shape(H, NB, M)) {
+    const size_t few = align_up(kCounterBytes) + few_tokens_workspace(H, NB, M, k);
+    if (few > off) off = few;
+  }
   return off;
 }
 
@@ -861,6 +865,19 @@ int nsmlp_prefill_slots_f16(const nsmlp_slot_table* table, const void* x, int M,
   char* base = (char*)ws;
   p.d.status = (int*)(base + kStatusOff);
   p.d.qbs_shift = __builtin_ctz((unsigned)p.d.qbs);
+  if (few_tokens_fit(p.d, M)) {
+    FewTokArgs f;
+    memset(&f, 0, sizeof(f));
+    f.d = p.d;
+    f.x = (const uint16_t*)x;
+    f.M = M;
+    f.sel = sel;
+    f.k = k;
+    f.out = (uint16_t*)out;
+    f.report_range = (long long)M * k < 2LL * p.d.NB;
+    launch_few_tokens(f, base + align_up(kCounterBytes), (hipStream_t)stream);
+    return check_launch("prefill");
+  }
   p.x = (const uint16_t*)x;
   p.M = M;
   p.sel = sel;

@@ -788,6 +788,31 @@ struct PrefillArgs {
 void launch_prefill(const PrefillArgs& p, hipStream_t s);
 int prefill_gu_check();  // NSMLP_OK, or the error (static LDS in the gate/up kernel)
 
+// The sparse MLP of a few tokens (at most 32), each with its own blocks, over
+// their union.
+struct FewTokArgs {
+  DecodeArgs d;           // slot table views, H, qbs, NB, code books, dq state, status, down_bias
+  const uint16_t* x;      // [M][H] fp16
+  int M;
+  const int32_t* sel;     // [M][k] block ids
+  int k;
+  uint16_t* out;          // [M][H] fp16
+  int report_range;       // report down products outside the fixed-point range
+  // set by launch_few_tokens: workspace and tiling
+  int NT, wgs;            // 16-token tiles, workgroups of the products
+  int32_t* nu;            // [2] union blocks, groups of the down's partial sums
+  int32_t* ublk;          // [NB] their ids, ascending
+  uint32_t* umask;        // [NB] their tokens
+  uint16_t* act;          // [M][NB 32] fp16, columns in union order
+  float* part;            // [groups][M][H] fp32
+  int gu_cw, gu_cgs;      // gate/up column waves of a workgroup, column groups
+  int gu_a2bytes, dn_a2bytes;
+};
+bool few_tokens_shape(int H, int NB, int M);  // what the workspace sizes depend on
+bool few_tokens_fit(const DecodeArgs& d, int M);
+size_t few_tokens_workspace(int H, int NB, int M, int k);
+void launch_few_tokens(const FewTokArgs& p, void* ws, hipStream_t s);
+
 // Dense-guard prefill MLP: every block for every token (M tokens) over a slot
 // table, as staged GEMMs on MFMA.  H % 256 == 0, NB % 4 == 0.
 struct DenseGuardArgs {

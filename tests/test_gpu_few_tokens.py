@@ -1,0 +1,105 @@
+"""Prefill calls of at most 32 tokens (the few-token kernels) against the
+oracle, over the edges of their tiling: one token, a full and an overfull
+16-token tile, hidden sizes whose 128-column chunks fill the column waves
+exactly, partly and over two column groups, unions smaller than a chunk of
+four blocks and larger than one batch of tile sums, host copies, duplicates
+and invalid ids.  Bars as in the prefill tests: relL2(gpu, exact) <=
+max(1e-3, e_ref) per token row, e_ref the fallback restatement's own error."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _u16(t):
+    return t.detach().cpu().contiguous().view(torch.int16).numpy().view(np.uint16)
+
+
+def _np(t):
+    return t.detach().cpu().contiguous().numpy()
+
+
+def _check(orc, L, x, sel, out, what):
+    """Every row of out against the oracle over the row's distinct blocks."""
+    y = _np(out).astype(np.float64)
+    for r in range(x.shape[0]):
+        blocks = np.unique(sel[r][(sel[r] >= 0) & (sel[r] < L.NB)])
+        gp, ga = orc.gather_rows_blocks(_np(L.gate_packed), _np(L.gate_absmax), blocks, L.H, L.qbs)
+        upk, ua = orc.gather_rows_blocks(_np(L.up_packed), _np(L.up_absmax), blocks, L.H, L.qbs)
+        dp, da = orc.gather_down_columns(_np(L.down_packed), _np(L.down_absmax), blocks, L.H, L.I, L.qbs)
+        local = np.arange(len(blocks), dtype=np.int32).reshape(1, -1)
+        ye, yf = orc.sparse_mlp(_u16(x[r:r + 1]), local, gp, ga, upk, ua, dp, da, qbs=L.qbs)
+        e_ref = orc.rel_l2(orc.f16_bits_to_f32(yf[0]).astype(np.float64), ye[0])
+        e_gpu = orc.rel_l2(y[r], ye[0])
+        assert e_gpu <= max(1e-3, e_ref), (what, r, e_gpu, e_ref)
+
+
+@pytest.mark.parametrize("H,I,M,k,qbs,dq", [
+    (256, 256, 1, 1, 64, False),       # 2 chunks of one wave, one block
+    (256, 1024, 16, 3, 128, True),
+    (1280, 2048, 17, 5, 64, True),     # 10 chunks over 2 column waves, second token tile
+    (2304, 2176, 5, 9, 64, False),     # 18 chunks over 4 column waves, 68 blocks
+    (5120, 1024, 12, 20, 64, True),    # 40 chunks over 8 column waves
+    (9216, 512, 16, 9, 64, True),      # 72 chunks: two column groups
+    (16384, 1024, 32, 11, 256, False),  # two token tiles over four column groups
+    (512, 32768, 32, 200, 64, True),   # 1024 blocks: several batches of tile sums a workgroup
+])
+def test_few_tokens_match_oracle(gpu, orc, H, I, M, k, qbs, dq):
+    from next_step_ai_amd.synth import make_synthetic_layer, synth_normal_f16
+
+    print(f"few tokens H={H} I={I} M={M} k={k} qbs={qbs} dq={dq}", flush=True)
+    L = make_synthetic_layer(H=H, I=I, R=16, seed=H + M, device=gpu, qbs=qbs, double_quant=dq)
+    x = synth_normal_f16(900 + M, (M, H), 1.0, gpu)
+    t = L.slot_table()
+    sel = L.router().route(x, k)
+    out = t.prefill(x, sel, check=True)
+    assert torch.equal(out, t.prefill(x, sel)), "not deterministic"
+    if dq:
+        assert torch.equal(out, L.slot_table(absmax="f32").prefill(x, sel))
+    _check(orc, L, x, _np(sel).astype(np.int64), out, f"H={H} M={M}")
+
+
+def test_few_tokens_host_copies_duplicates_and_invalid_ids(gpu, orc):
+    """Half of the blocks in host copies: the same bits as all resident; a
+    repeated id counts once; an id out of range is reported and adds nothing."""
+    from next_step_ai_amd.synth import make_synthetic_layer, synth_normal_f16
+
+    H, I, M, k = 1024, 2048, 20, 6
+    L = make_synthetic_layer(H=H, I=I, R=16, seed=5, device=gpu, double_quant=True)
+    x = synth_normal_f16(6, (M, H), 1.0, gpu)
+    sel = _np(L.router().route(x, k)).copy()
+    sel[3, 2] = sel[3, 1]
+    for absmax in ("dq", "f32"):
+        full = L.slot_table(absmax=absmax)
+        out = full.prefill(x, torch.from_numpy(sel).to(gpu), check=True)
+        resident = torch.arange(0, L.NB, 2, dtype=torch.int32)
+        part = L.slot_table(resident_blocks=resident, host_copy=True, absmax=absmax)
+        assert torch.equal(part.prefill(x, torch.from_numpy(sel).to(gpu), check=True), out)
+    _check(orc, L, x, sel.astype(np.int64), out, "duplicates")
+    bad = sel.copy()
+    bad[7, 0], bad[8, 5] = -1, L.NB + 3
+    with pytest.raises(RuntimeError, match="out of range"):
+        full.prefill(x, torch.from_numpy(bad).to(gpu), check=True)
+    out_bad = full.prefill(x, torch.from_numpy(bad).to(gpu))
+    _check(orc, L, x, bad.astype(np.int64), out_bad, "invalid ids")
+
+
+def test_few_tokens_do_not_mix(gpu):
+    """A token with an infinity leaves every other token's output as it is,
+    also where they share blocks."""
+    from next_step_ai_amd.synth import make_synthetic_layer, synth_normal_f16
+
+    H, I, M = 1024, 1024, 9
+    L = make_synthetic_layer(H=H, I=I, R=16, seed=8, device=gpu)
+    t = L.slot_table()
+    x = synth_normal_f16(9, (M, H), 1.0, gpu)
+    sel = torch.arange(8, dtype=torch.int32, device=gpu).repeat(M, 1)
+    sel[4] += 4
+    out = t.prefill(x, sel)
+    x2 = x.clone()
+    x2[4, 100] = float("inf")
+    out2 = t.prefill(x2, sel)
+    others = [r for r in range(M) if r != 4]
+    assert torch.equal(out2[others], out[others])
+    assert not torch.isfinite(out2[4].float()).all()
