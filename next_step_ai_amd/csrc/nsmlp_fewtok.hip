@@ -32,10 +32,13 @@
 //
 // Every sum is taken in a fixed order.
 //
-// At hidden 16384 and 8 tokens (1092 of 1664 blocks, 894 MB) gate/up and down
-// take about 240 us, 3.7 TB/s: two waves a SIMD (the tokens' registers) leave
-// the lookups' and MFMAs' latency partly open, not the weight stream.
+// At hidden 16384 and 8 tokens (1092 of 1664 blocks, 894 MB) gate/up takes 146
+// us (4.0 TB/s) and down 91 (3.2 TB/s): two waves a SIMD (the tokens'
+// registers) leave the lookups' and MFMAs' latency partly open (without the
+// weight loads gate/up still takes 133 us); the loads are temporal, as a row's
+// 128-byte line serves two chunks (172 -> 158 us against nontemporal ones).
 #include <mutex>
+#include <utility>
 
 #include "nsmlp_replut.h"
 
@@ -76,6 +79,9 @@ __device__ __forceinline__ void group_values(float v, float (&o)[4]) {
 }
 __device__ __forceinline__ uint32_t ft_lane(uint32_t v, int lane) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+}
+__device__ __forceinline__ uint64_t ft_lane64(uint64_t v, int lane) {
+  return ((uint64_t)ft_lane((uint32_t)(v >> 32), lane) << 32) | ft_lane((uint32_t)v, lane);
 }
 // 8 codes of a packed dword as fp16, in element order.
 __device__ __forceinline__ half8_t ft_codes8(uint32_t v, uint32_t (&ad)[4]) {
@@ -165,6 +171,7 @@ __global__ void __launch_bounds__(1024) k_ft_list(FewTokArgs p) {
 // hands each to all four groups.
 template <int NT, int NCH>
 struct FtGeo {
+  static constexpr bool kPipe = NT == 1 && NCH <= 6;  // the chunks' own pipeline (see below)
   static constexpr int SU = (NCH + 1) / 2;  // chunks of a tile's first unit (the second has NCH - SU)
   static constexpr int PD = 8 / (SU == 3 ? 4 : SU);  // units in flight: 8 chunk loads (6 for SU = 3)
   static constexpr int RB = PD / 2;                  // tiles per loop body
@@ -203,24 +210,15 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
   }
   lds_barrier();
   const rsrc_t rx = make_rsrc(p.x, M * H * 2);
-  // What issue needs of the kernel arguments, kept in SGPRs (opaque to the
-  // compiler, which otherwise loads the fields again for every tile: a scalar
-  // load's round trip each, waited for together with the LDS reads).
-  auto bytes_of = [](const auto* q) { return reinterpret_cast<uint64_t>(q); };
-  auto pick = [](bool c, auto a, auto b) { return c ? a : b; };  // by value: a conditional over the variables selects an address
-  uint64_t w_g = bytes_of(d.gate.packed), w_u = bytes_of(d.up.packed), w_hg = bytes_of(d.host_gate.packed),
-           w_hu = bytes_of(d.host_up.packed);
-  uint64_t a_g = DQ ? bytes_of(d.gate.qabsmax) : bytes_of(d.gate.absmax);
-  uint64_t a_u = DQ ? bytes_of(d.up.qabsmax) : bytes_of(d.up.absmax);
-  uint64_t a_hg = DQ ? bytes_of(d.host_gate.qabsmax) : bytes_of(d.host_gate.absmax);
-  uint64_t a_hu = DQ ? bytes_of(d.host_up.qabsmax) : bytes_of(d.host_up.absmax);
-  uint64_t s_g = bytes_of(d.gate.absmax2), s_u = bytes_of(d.up.absmax2);
+  // opaque to the compiler, which otherwise loads the fields again for every
+  // tile (a scalar load's round trip, waited for together with the LDS reads)
   uint32_t rs = (uint32_t)d.gate.row_stride, A = (uint32_t)d.gate.abs_row_stride;
   uint32_t qsh = (uint32_t)d.qbs_shift, dsh = (uint32_t)d.dq_shift;
+  uint64_t s_g = reinterpret_cast<uint64_t>(d.gate.absmax2), s_u = reinterpret_cast<uint64_t>(d.up.absmax2);
   float off_g = d.gate.offset, off_u = d.up.offset;
-  asm volatile(""
-               : "+s"(w_g), "+s"(w_u), "+s"(w_hg), "+s"(w_hu), "+s"(a_g), "+s"(a_u), "+s"(a_hg), "+s"(a_hu), "+s"(s_g),
-                 "+s"(s_u), "+s"(rs), "+s"(A), "+s"(qsh), "+s"(dsh), "+s"(off_g), "+s"(off_u));
+  asm volatile("" : "+s"(rs), "+s"(A), "+s"(qsh), "+s"(dsh), "+s"(s_g), "+s"(s_u), "+s"(off_g), "+s"(off_u));
+  // by value: a conditional over the variables themselves selects an address
+  auto pick = [](bool c, auto a, auto b) { return c ? a : b; };
 
   struct Stage {
     uint4 w[SU];
@@ -230,52 +228,53 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
   for (int pb = p_lo; pb < p_hi; pb += G::kSlots / 2) {
     const int np = min(p_hi - pb, G::kSlots / 2), ntl = 2 * np;
     const int R = (ntl + RW - 1) / RW, VT = R * CGS;
-    // lane i: block reference of pair i (slot, or the block id with bit 30 for
-    // a host copy; bit 31: unavailable)
-    uint32_t enc_v = 0x80000000u, bid_v = 0;
-    if (lane < np) {
-      const int b = p.ublk[(pb + lane) >> 1];
-      const BlockRef br = resolve_id(d, b);
-      enc_v = !br.ok ? 0x80000000u : br.dev ? (uint32_t)br.q : (0x40000000u | (uint32_t)br.q);
-      bid_v = (uint32_t)b;
-      if (!br.ok && wave == 0) atomicOr(d.status, NSMLP_STATUS_BLOCK_UNAVAILABLE);
+    // lane t: tile t's packed rows and its block's absmax (addresses), the
+    // flat index of its first absmax; bit 31 of that: the block is unavailable
+    uint64_t tw = 0, ta = 0;
+    uint32_t tf = 0x80000000u;
+    if (lane < ntl) {
+      const int pi = pb + (lane >> 1), h16 = (pi & 1) * 16;
+      const bool up = (lane & 1) != 0;
+      const BlockRef br = resolve_id(d, p.ublk[pi >> 1]);
+      if (br.ok) {
+        const ProjView& pv = up ? (br.dev ? d.up : d.host_up) : (br.dev ? d.gate : d.host_gate);
+        tw = reinterpret_cast<uint64_t>(pv.packed + br.q * pv.blk_stride + (long long)h16 * rs);
+        ta = DQ ? reinterpret_cast<uint64_t>(pv.qabsmax + br.q * pv.abs_blk_stride + (long long)h16 * A)
+                : reinterpret_cast<uint64_t>(pv.absmax + br.q * pv.abs_blk_stride + (long long)h16 * A);
+        tf = (32u * (uint32_t)br.b + (uint32_t)h16) * A;
+      } else if (wave == 0) {
+        atomicOr(d.status, NSMLP_STATUS_BLOCK_UNAVAILABLE);
+      }
     }
     int icg = 0, ir = 0;  // column group and round of the next tile to issue
     auto issue = [&](Stage& st, auto unit) {
       constexpr int U = decltype(unit)::value;
       const int t = ir * RW + rw;
       const bool live = icg < CGS && t < ntl;
-      const int lp = live ? t >> 1 : 0;
-      const uint32_t enc = ft_lane(enc_v, lp);
-      const bool up = (t & 1) != 0, dev = (enc & 0x40000000u) == 0;
-      const bool ok = live && (enc & 0x80000000u) == 0;
-      const uint32_t q = ok ? enc & 0x3FFFFFFFu : 0u;
-      const uint32_t h16 = (uint32_t)((pb + lp) & 1) * 16u;
+      const int l = live ? t : 0;
+      const uint32_t f = ft_lane(tf, l);
+      const bool ok = live && (int)f >= 0;
       const int chb = (icg * CW + cw) * NCH;
-      const uint64_t base = pick(up, pick(dev, w_u, w_hu), pick(dev, w_g, w_hg)) + (uint64_t)q * (32u * rs) + h16 * rs;
-      const rsrc_t rp = make_rsrc(reinterpret_cast<const void*>(base), ok ? 16 * (int)rs : 0);
-      // columns past the last chunk read the next row (or zeros past the
-      // tile): their tokens are zero
+      const rsrc_t rp = make_rsrc(reinterpret_cast<const void*>(ft_lane64(tw, l)), ok ? 16 * (int)rs : 0);
+      // temporal: a row's 128-byte line serves two chunks.  Columns past the
+      // last chunk read the next row (or zeros past the tile): their tokens
+      // are zero
       const uint32_t voff = (uint32_t)j * rs + (uint32_t)(chb * 64) + 16u * (uint32_t)g;
       constexpr int c0 = U == 0 ? 0 : SU, c1 = U == 0 ? SU : NCH;
 #pragma unroll
-      for (int c = c0; c < c1; ++c) st.w[c - c0] = buf_ld16(rp, voff + 64u * (uint32_t)c, 0);
-      {
-        const uint64_t ab = pick(up, pick(dev, a_u, a_hu), pick(dev, a_g, a_hg)) + (uint64_t)q * (32u * A * (DQ ? 1u : 4u));
-        const rsrc_t ra = make_rsrc(reinterpret_cast<const void*>(ab), ok ? (int)(32u * A * (DQ ? 1u : 4u)) : 0);
-        const rsrc_t r2 = make_rsrc(reinterpret_cast<const void*>(pick(up, s_u, s_g)), ok ? p_a2 : 0);
-        const uint32_t r = h16 + (uint32_t)j, bid = ft_lane(bid_v, lp);
-        const uint32_t f0 = (32u * bid + r) * A;
+      for (int c = c0; c < c1; ++c) st.w[c - c0] = buf_ld16c(rp, voff + 64u * (uint32_t)c, 0);
+      const rsrc_t ra = make_rsrc(reinterpret_cast<const void*>(ft_lane64(ta, l)), ok ? (int)(16u * A * (DQ ? 1u : 4u)) : 0);
+      const rsrc_t r2 = make_rsrc(reinterpret_cast<const void*>(pick((t & 1) != 0, s_u, s_g)), ok ? p_a2 : 0);
 #pragma unroll
-        for (int i = 0; i < (2 * (c1 - c0) + 3) / 4; ++i) {
-          const uint32_t e = (uint32_t)(128 * chb + 64 * (2 * c0 + 4 * i + g)) >> qsh;
-          if constexpr (DQ) {
-            st.qa[i] = buf_ldu8(ra, ((r >> 1) * A + e) * 2u + (r & 1u), 0);
-            st.am[i] = buf_ldfc(r2, ((f0 + e) >> dsh) * 4u, 0);
-          } else {
-            st.qa[i] = 0;
-            st.am[i] = buf_ldf(ra, (r * A + e) * 4u, 0);
-          }
+      for (int i = 0; i < (2 * (c1 - c0) + 3) / 4; ++i) {
+        const uint32_t e = (uint32_t)(128 * chb + 64 * (2 * c0 + 4 * i + g)) >> qsh;
+        if constexpr (DQ) {
+          // codes of rows 2 i and 2 i + 1 are interleaved
+          st.qa[i] = buf_ldu8c(ra, (uint32_t)(j & 14) * A + 2u * e + (uint32_t)(j & 1), 0);
+          st.am[i] = buf_ldfc(r2, ((f + (uint32_t)j * A + e) >> dsh) * 4u, 0);
+        } else {
+          st.qa[i] = 0;
+          st.am[i] = buf_ldfc(ra, ((uint32_t)j * A + e) * 4u, 0);
         }
       }
       if constexpr (U == 1) {
@@ -310,67 +309,113 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
     }
     sched_fence();
 
+    // With up to 6 chunks a wave the registers allow a pipeline of the chunks
+    // (kPipe): chunk c + 1's lookups go out before chunk c's MFMAs, and the
+    // absmax multiplies chunk c - 1's results after them (16 lookups and their
+    // address moves and the MFMAs of a chunk lie between an MFMA and the first
+    // read of its result; the last chunk of a tile has the drain instead).
+    // With more, a chunk's lookups, MFMAs, drain and scaling follow each other.
     uint32_t ad[4];
+    auto set_ad = [&](int t) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) ad[m] = ((t & 1) ? 128u : 0u) + (uint32_t)(lane & 31) * 4u;
+    };
+    auto lookup = [&](half8_t (&b)[4], uint4 w) {
+      swap32(w.x, w.z);
+      swap32(w.y, w.w);
+      b[0] = ft_codes8(w.x, ad);
+      b[1] = ft_codes8(w.y, ad);
+      b[2] = ft_codes8(w.z, ad);
+      b[3] = ft_codes8(w.w, ad);
+    };
+    half8_t bq[2][4];
+    set_ad(rw);
+    if constexpr (G::kPipe) lookup(bq[0], st[0].w[0]);
     int cg = 0, r = 0;
     for (int v0 = 0; v0 < VT; v0 += RB) {
 #pragma unroll
       for (int i = 0; i < RB; ++i) {
         if (v0 + i < VT) {  // uniform over the workgroup
           if (r == 0 && v0 + i > 0) load_x(cg);
-          const int t = r * RW + rw;
+          const int t = r * RW + rw, tn = (r + 1 < R ? r + 1 : 0) * RW + rw;
           const int mych = min(chunks - (cg * CW + cw) * NCH, NCH);
-          const bool ok = t < ntl && (ft_lane(enc_v, t < ntl ? t >> 1 : 0) & 0x80000000u) == 0;
-#pragma unroll
-          for (int m = 0; m < 4; ++m) ad[m] = ((t & 1) ? 128u : 0u) + (uint32_t)(lane & 31) * 4u;
-          float4_t acc[NT];
+          const bool ok = t < ntl && (int)ft_lane(tf, t < ntl ? t : 0) >= 0;
+          float4_t acc[NT], cc[2][2][NT];
 #pragma unroll
           for (int n = 0; n < NT; ++n) acc[n] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-          auto unit = [&](Stage& su, auto uc) {
-            constexpr int U = decltype(uc)::value;
-            constexpr int c0 = U == 0 ? 0 : SU, c1 = U == 0 ? SU : NCH;
+          // absmax of the lane's halves (lane group g: halves 4 q + g of a unit)
+          auto resolve = [&](float (&o)[NH], const Stage& su, int first, int count) {
 #pragma unroll
-            for (int cp = c0; cp < c1; cp += 2) {  // two chunks: four halves, one absmax load of the lane
-              constexpr int kPair = 2;
-              float4_t cc[2 * kPair][NT];
-#pragma unroll
-              for (int c = cp; c < cp + 2 && c < c1; ++c) {
-                uint4 w = su.w[c - c0];
-                swap32(w.x, w.z);
-                swap32(w.y, w.w);
-                const uint32_t dw[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                  const half8_t b = ft_codes8(dw[s], ad);
-                  float4_t(&o)[NT] = cc[2 * (c - cp) + (s >> 1)];
-#pragma unroll
-                  for (int n = 0; n < NT; ++n)
-                    o[n] = mfma16(x[c][s][n], b, (s & 1) ? o[n] : float4_t{0.0f, 0.0f, 0.0f, 0.0f});
-                }
-              }
-              // the halves' absmax, every one in all lane groups
-              const int q = (cp - c0) / 2;
+            for (int q = 0; q < (2 * count + 3) / 4; ++q) {
               float a = su.am[q];
               if constexpr (DQ) a = dq_absmax(c2[((t & 1) ? 256 : 0) + su.qa[q]], a, pick((t & 1) != 0, off_u, off_g));
-              a = ok && 2 * cp + g < 2 * mych ? a : 0.0f;
-              float am[4];
-              group_values(a, am);
-              mfma_drain();
-#pragma unroll
-              for (int hb = 0; hb < 4 && cp + hb / 2 < c1; ++hb)
-#pragma unroll
-                for (int n = 0; n < NT; ++n)
-#pragma unroll
-                  for (int e = 0; e < 4; ++e) acc[n][e] = __builtin_fmaf(cc[hb][n][e], am[hb], acc[n][e]);
-#pragma unroll
-              for (int n = 0; n < NT; ++n) asm volatile("" : "+v"(acc[n]));  // summed here, not at its use
+              o[q] = ok && 2 * first + 4 * q + g < 2 * mych ? a : 0.0f;
             }
           };
-          unit(st[2 * i], U0{});
-          issue(st[2 * i], U0{});
-          sched_fence();
-          unit(st[2 * i + 1], U1{});
-          issue(st[2 * i + 1], U1{});
-          sched_fence();
+          float ar[NH], am[4];
+          resolve(ar, st[2 * i], 0, SU);
+          auto scale = [&](auto cc_) {
+            constexpr int c = decltype(cc_)::value;
+            constexpr int h = 2 * (c < SU ? c : c - SU);  // the chunk's first half in its unit
+            if constexpr (h % 4 == 0) group_values(ar[h / 4], am);
+#pragma unroll
+            for (int hb = 0; hb < 2; ++hb)
+#pragma unroll
+              for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[n][e] = __builtin_fmaf(cc[G::kPipe ? c & 1 : 0][hb][n][e], am[(h + hb) % 4], acc[n][e]);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) asm volatile("" : "+v"(acc[n]));  // summed here, not at its use
+          };
+          auto products = [&](auto cc_, const half8_t (&b)[4]) {
+            constexpr int c = decltype(cc_)::value, o = G::kPipe ? c & 1 : 0;
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+              for (int n = 0; n < NT; ++n)
+                cc[o][s >> 1][n] = mfma16(x[c][s][n], b[s], (s & 1) ? cc[o][s >> 1][n] : float4_t{0.0f, 0.0f, 0.0f, 0.0f});
+          };
+          auto chunk = [&](auto cc_) {
+            constexpr int c = decltype(cc_)::value;
+            if constexpr (G::kPipe) {
+              if constexpr (c + 1 < NCH) {
+                lookup(bq[(c + 1) & 1], c + 1 < SU ? st[2 * i].w[c + 1] : st[2 * i + 1].w[c + 1 - SU]);
+              } else {
+                set_ad(tn);
+                lookup(bq[(c + 1) & 1], st[(2 * i + 2) % PD].w[0]);
+              }
+              sched_fence();
+              products(cc_, bq[c & 1]);
+              sched_fence();
+              if constexpr (c > 0) {
+                scale(std::integral_constant<int, (c > 0 ? c - 1 : 0)>{});
+                if constexpr (c == SU) resolve(ar, st[2 * i + 1], SU, NCH - SU);
+              }
+              if constexpr (c == SU - 1) issue(st[2 * i], U0{});
+              if constexpr (c == (NCH - 2 > SU ? NCH - 2 : SU)) issue(st[2 * i + 1], U1{});
+              if constexpr (c == NCH - 1) {
+                mfma_drain();
+                scale(cc_);
+              }
+            } else {
+              if constexpr (c == 0) set_ad(t);
+              if constexpr (c == SU) resolve(ar, st[2 * i + 1], SU, NCH - SU);
+              lookup(bq[0], c < SU ? st[2 * i].w[c] : st[2 * i + 1].w[c - SU]);
+              products(cc_, bq[0]);
+              mfma_drain();
+              scale(cc_);
+              if constexpr (c == SU - 1) issue(st[2 * i], U0{});
+              if constexpr (c == NCH - 1) issue(st[2 * i + 1], U1{});
+            }
+            sched_fence();
+          };
+          [&]<int... C>(std::integer_sequence<int, C...>) {
+            (chunk(std::integral_constant<int, C>{}), ...);
+          }(std::make_integer_sequence<int, NCH>{});
+          if constexpr (G::kPipe && NCH % 2 != 0) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) bq[0][s] = bq[1][s];
+          }
           // the column waves' sums: one wave per (row wave, token tile), a
           // different one each round, adds them in column order
           const int par = (v0 + i) & 1;
@@ -651,12 +696,13 @@ template <bool DQ, bool HOST, int NT>
 constexpr FtKernel ft_down() {
   return FtKernel{k_ft_down<DQ, HOST, NT>, FdGeo<NT>::kLds};
 }
-// [dq][chunks - 5 of one token tile; 4 + chunks - 3 of two]
+// [dq][one token tile of 4, 5, 6, 8 chunks, two of 3, 4]
 const FtKernel kFtGu[2][6] = {
-    {ft_gu<false, 1, 5>(), ft_gu<false, 1, 6>(), ft_gu<false, 1, 7>(), ft_gu<false, 1, 8>(), ft_gu<false, 2, 3>(),
+    {ft_gu<false, 1, 4>(), ft_gu<false, 1, 5>(), ft_gu<false, 1, 6>(), ft_gu<false, 1, 8>(), ft_gu<false, 2, 3>(),
      ft_gu<false, 2, 4>()},
-    {ft_gu<true, 1, 5>(), ft_gu<true, 1, 6>(), ft_gu<true, 1, 7>(), ft_gu<true, 1, 8>(), ft_gu<true, 2, 3>(),
+    {ft_gu<true, 1, 4>(), ft_gu<true, 1, 5>(), ft_gu<true, 1, 6>(), ft_gu<true, 1, 8>(), ft_gu<true, 2, 3>(),
      ft_gu<true, 2, 4>()}};
+constexpr int kFtGuChunks[6] = {4, 5, 6, 8, 3, 4};
 // [dq][host copies][token tiles - 1]
 const FtKernel kFtDown[2][2][2] = {{{ft_down<false, false, 1>(), ft_down<false, false, 2>()},
                                     {ft_down<false, true, 1>(), ft_down<false, true, 2>()}},
@@ -680,20 +726,28 @@ void ft_launch(const FtKernel& k, int wgs, const FewTokArgs& p, hipStream_t s) {
   k.fn<<<dim3((unsigned)wgs), dim3(kFtThreads), k.lds, s>>>(p);
 }
 
-// Chunks a wave holds and the column waves of a workgroup for H columns: the
-// fewest column groups (each a pass over the workgroup's tiles with its own
-// tokens in registers), then the fewest chunks a wave, then the fewest
-// column waves.
-void ft_columns(int H, int NT, int* nch, int* cw, int* cgs) {
-  const int chunks = H / 128, top = 8 / NT, low = NT == 1 ? 5 : 3;
-  const int waves = (chunks + top - 1) / top;
-  *cgs = (waves + kFtWaves - 1) / kFtWaves;
-  const int per = (chunks + *cgs - 1) / *cgs;
-  int w = 1;
-  while (w < kFtWaves && w * top < per) w *= 2;
-  *cw = w;
-  int n = (per + w - 1) / w;
-  *nch = n < low ? low : n;
+// The kernel (by the chunks a wave holds), column waves of a workgroup and
+// column groups (each a pass over the workgroup's tiles with its own tokens in
+// registers) for H columns: the fewest column groups, then the fewest chunk
+// slots, then the fewest chunks a wave (hidden 16384, 8 tokens: 8 chunks x 8
+// waves x 2 groups 146 us, 4 x 8 x 4 155, 6 x 8 x 3 177; hidden 4096, 12
+// tokens: 4 x 8 waves 23.1 us, 8 x 4 25.8; two token tiles at hidden 16384: 4
+// chunks 290 us, 3 chunks 350).
+int ft_columns(int H, int NT, int* cw, int* cgs) {
+  const int chunks = H / 128;
+  int best = 0, cost = 0x7FFFFFFF;
+  for (int i = NT == 1 ? 0 : 4; i < (NT == 1 ? 4 : 6); ++i)
+    for (int w = 1; w <= kFtWaves; w *= 2) {
+      const int n = kFtGuChunks[i], c = (chunks + w * n - 1) / (w * n);
+      const int v = c * 100000 + c * n * w * 16 + n;
+      if (v < cost) {
+        cost = v;
+        best = i;
+        *cw = w;
+        *cgs = c;
+      }
+    }
+  return best;
 }
 
 }  // namespace
@@ -739,13 +793,12 @@ void launch_few_tokens(const FewTokArgs& args, void* ws, hipStream_t s) {
   p.act = (uint16_t*)w;
   w += up((size_t)p.M * d.NB * 64);
   p.part = (float*)w;
-  int nch;
-  ft_columns(d.H, NT, &nch, &p.gu_cw, &p.gu_cgs);
+  const int gu = ft_columns(d.H, NT, &p.gu_cw, &p.gu_cgs);
   const long long n2 = (((long long)d.H * d.NB * 32 / d.qbs) + (1LL << d.dq_shift) - 1) >> d.dq_shift;
   p.gu_a2bytes = p.dn_a2bytes = (int)(n2 * 4);
   k_ft_list<<<dim3(1), dim3(1024), 0, s>>>(p);
   ft_set_lds();
-  ft_launch(kFtGu[d.dq ? 1 : 0][NT == 1 ? nch - 5 : 4 + nch - 3], cus, p, s);
+  ft_launch(kFtGu[d.dq ? 1 : 0][gu], cus, p, s);
   ft_launch(kFtDown[d.dq ? 1 : 0][d.host_down.packed != nullptr ? 1 : 0][NT - 1], cus, p, s);
   const long long n = (long long)p.M * d.H;
   k_ft_fin<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(p);
