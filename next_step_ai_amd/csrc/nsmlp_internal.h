@@ -701,6 +701,7 @@ struct DecodeArgs {
   int st_gu_rounds;      // gate/up rounds per workgroup
   int st_dn_gx;          // down workgroups per 64-row chunk (block groups)
   int st_dn_per;         // blocks per down wave (<= 64)
+  int st_dn_rows;        // the down weight is row-major (its own form of the down kernel)
   int st_gu_bytes;       // extent of one gate/up slot: packed bytes, absmax bytes
   int st_gu_abytes;
   int st_dn_bytes;       // extent of one down block: packed bytes, absmax bytes

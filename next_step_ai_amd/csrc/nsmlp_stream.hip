@@ -71,6 +71,13 @@ constexpr size_t kGuSelLds = (size_t)kGuSelWord * 4 + kSelMaxK * sizeof(int32_t)
 constexpr size_t kDnLds = kRepLutBytes + kMaxDnBlocks * 16 * 4 + kMaxDnBlocks * 4 + kWaves * kWave * 4;
 constexpr int kDnA2Max = 1024;
 constexpr size_t kDnDqLds = kDnLds + (256 + kDnA2Max) * sizeof(float);
+// row-major rows: also a tile per wave, 64 rows of 4 blocks (16 packed bytes
+// and an absmax each) at row strides that spread a column over the banks
+constexpr int kDnTileBlocks = 4;
+constexpr int kDnTileRow = 16 * kDnTileBlocks + 16, kDnTileAbsRow = 4 * kDnTileBlocks + 4;  // bytes
+constexpr int kDnTile = kWave * (kDnTileRow + kDnTileAbsRow);
+constexpr size_t kDnRowsLds = kDnLds + kWaves * kDnTile;
+static_assert(kDnRowsLds <= 160 * 1024, "LDS");
 
 // Encoded block reference: < 2^30 -> HBM slot; bit 30 -> host copy of the
 // block id in the low bits; bit 31 -> invalid (zero contribution).
@@ -451,6 +458,10 @@ __global__ void __launch_bounds__(kThreads8, 2) k_gu_rep(DecodeArgs args) {
   }
 }
 
+struct DnTile {
+  uint4 w[4];
+  float am[4];
+};
 struct DnStage {
   uint4 w[2];
   float am[2];     // absmax (fp32 absmax storage)
@@ -529,7 +540,15 @@ __device__ __forceinline__ void pin_dn_rest(DecodeArgs& a) {
   a.outpart = (float*)outpart;
 }
 
-template <bool DQ>
+// ROWS: the down weight is row-major (row o holds its blocks' 16 packed bytes
+// one after the other, and their absmax), as a runtime that gathers a token's
+// blocks has it.  A lane's row read 16 bytes at a time, as the block-major
+// form does, would fetch a 64-row column of lines for every block, and most of
+// them several times; a wave therefore reads tiles of 4 blocks, 4 lanes to a
+// row (64 contiguous bytes), and turns them into rows per lane through LDS of
+// its own (hidden 16384, 208 blocks, 68 MB: 77.5 -> 28 us).  The sums and
+// their order are those of the block-major form, bit for bit.
+template <bool DQ, bool ROWS>
 __global__ void __launch_bounds__(kThreads8, 2) k_down_rep(DecodeArgs args) {
   DecodeArgs a = args;
   pin_dn_first(a);
@@ -607,8 +626,29 @@ __global__ void __launch_bounds__(kThreads8, 2) k_down_rep(DecodeArgs args) {
   pin_dn_rest<DQ>(a);
   if (lane >= nbv) enc_v = kBad;
   DnStage st[kDnStages];
+  DnTile tile[kDnStages];
+  [[maybe_unused]] const rsrc_t rrp = make_rsrc(a.down.packed, a.st_dn_bytes), rra = make_rsrc(a.down.absmax, a.st_dn_abytes);
+  auto tile_issue = [&](DnTile& tl, int t) {
+    // lane: block 4 t + lane % 4 of rows 16 i + lane / 4
+    const int jj = kDnTileBlocks * t + (lane & 3);
+    const uint32_t e = (uint32_t)__shfl((int)enc_v, jj & 63, kWave);
+    const bool ok = jj < nbv && !(e & kBad);
+    const uint32_t r0 = (uint32_t)(c * kWave + (lane >> 2));
+    const uint32_t rs = (uint32_t)a.down.row_stride, ars = (uint32_t)a.down.abs_row_stride;
+    const uint32_t vw = ok ? r0 * rs + e * 16u : kOffNone, va = ok ? (r0 * ars + e) * 4u : kOffNone;
 #pragma unroll
-  for (int i = 0; i < kDnStages; ++i) {
+    for (int i = 0; i < 4; ++i) {
+      // temporal: the rest of the row's lines is read by the next tiles
+      tl.w[i] = buf_ld16c(rrp, vw, 16u * i * rs);
+      tl.am[i] = buf_ldfc(rra, va, 64u * i * ars);
+    }
+  };
+  if constexpr (ROWS) {
+#pragma unroll
+    for (int i = 0; i < kDnStages; ++i) tile_issue(tile[i], i);
+  }
+#pragma unroll
+  for (int i = 0; i < (ROWS ? 0 : kDnStages); ++i) {
     const bool in = i < T;
     dn_issue<DQ>(a, in ? lane_value(enc_v, 2 * i) : kBad, roff, aoff, st[i].w[0], st[i].am[0], st[i].qa[0]);
     dn_issue<DQ>(a, in ? lane_value(enc_v, 2 * i + 1) : kBad, roff, aoff, st[i].w[1], st[i].am[1], st[i].qa[1]);
@@ -654,7 +694,40 @@ __global__ void __launch_bounds__(kThreads8, 2) k_down_rep(DecodeArgs args) {
   const uint32_t* wact = actp + jw0 * 16;
   const float* wscale = ascale + jw0;
   float acc = 0.0f;
-  for (int t0 = 0; t0 < T; t0 += kDnStages) {
+  if constexpr (ROWS) {
+    uint8_t* tw = reinterpret_cast<uint8_t*>(lds) + kDnLds + wave * kDnTile;
+    uint8_t* ta = tw + kWave * kDnTileRow;
+    const int TT = (nbv + kDnTileBlocks - 1) / kDnTileBlocks;
+    for (int t0 = 0; t0 < TT; t0 += kDnStages) {
+#pragma unroll
+      for (int i = 0; i < kDnStages; ++i) {
+        const int t = t0 + i;
+        // the wave's own tile: LDS operations of a wave are done in order
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          const int r = 16 * m + (lane >> 2), b = lane & 3;
+          *reinterpret_cast<uint4*>(tw + r * kDnTileRow + 16 * b) = tile[i].w[m];
+          *reinterpret_cast<float*>(ta + r * kDnTileAbsRow + 4 * b) = tile[i].am[m];
+        }
+        tile_issue(tile[i], t + kDnStages);
+        __builtin_amdgcn_wave_barrier();
+        uint4 w[kDnTileBlocks];
+        float am[kDnTileBlocks];
+#pragma unroll
+        for (int b = 0; b < kDnTileBlocks; ++b) {
+          w[b] = *reinterpret_cast<const uint4*>(tw + lane * kDnTileRow + 16 * b);
+          am[b] = *reinterpret_cast<const float*>(ta + lane * kDnTileAbsRow + 4 * b);
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int b = 0; b < kDnTileBlocks; ++b) {
+          const int jj = kDnTileBlocks * t + b;
+          if (jj < nbv) acc += rep_dot32(w[b], wact + jj * 16, ad) * (am[b] * wscale[jj]);
+        }
+      }
+    }
+  }
+  for (int t0 = 0; t0 < (ROWS ? 0 : T); t0 += kDnStages) {
 #pragma unroll
     for (int i = 0; i < kDnStages; ++i) {
       const int t = t0 + i;
@@ -923,6 +996,10 @@ bool plan_streaming(DecodeArgs& a, int cus) {
   if (nbw > kMaxDnBlocks) return false;
   GX = (a.k + nbw - 1) / nbw;
   const long long per = (nbw + kWaves - 1) / kWaves;
+  // row-major rows go through LDS tiles (every offset of the whole weight in
+  // 31 bits); single-block weights are the same in both layouts
+  a.st_dn_rows = !a.dq && a.host_down.packed == nullptr && a.down.blk_stride == 16 && a.down.abs_blk_stride == 1 &&
+                 a.down.row_stride > 16 && dn_bytes + a.down.row_stride < lim && dn_abytes + 4 * a.down.abs_row_stride < lim;
   a.cs = kSplit;
   a.splits = S;
   a.st_gu_rounds = (int)R;
@@ -931,8 +1008,8 @@ bool plan_streaming(DecodeArgs& a, int cus) {
   a.st_dn_per = (int)per;
   a.st_gu_bytes = (int)gu_bytes;
   a.st_gu_abytes = (int)gu_abytes;
-  a.st_dn_bytes = (int)dn_bytes;
-  a.st_dn_abytes = (int)dn_abytes;
+  a.st_dn_bytes = (int)(a.st_dn_rows ? dn_bytes + a.down.row_stride - 16 : dn_bytes);
+  a.st_dn_abytes = (int)(a.st_dn_rows ? dn_abytes + 4 * (a.down.abs_row_stride - 1) : dn_abytes);
   return true;
 }
 
@@ -950,8 +1027,9 @@ void launch_decode_streaming(const DecodeArgs& a, hipStream_t s) {
     for (int d = 0; d < 2; ++d)
       for (int f = 0; f < 2; ++f)
         for (int m = 0; m < 3; ++m) set_lds_limit(gu_fns[d][f][m], m ? kGuSelLds : (d ? kGuDqLds : kGuLds));
-    set_lds_limit(k_down_rep<false>, kDnLds);
-    set_lds_limit(k_down_rep<true>, kDnDqLds);
+    set_lds_limit(k_down_rep<false, false>, kDnLds);
+    set_lds_limit(k_down_rep<false, true>, kDnRowsLds);
+    set_lds_limit(k_down_rep<true, false>, kDnDqLds);
   });
   const bool affine = a.gate_bias != nullptr || a.up_bias != nullptr || a.mask != nullptr;
   const int mode = a.sel_scores == nullptr ? 0 : (a.NB <= 4 * kThreads8 ? 1 : 2);
@@ -960,9 +1038,11 @@ void launch_decode_streaming(const DecodeArgs& a, hipStream_t s) {
   gu<<<dim3(a.st_gu_wgs), dim3(kThreads8), gu_lds, s>>>(a);
   const dim3 gd((a.H / kWave) * a.st_dn_gx), bd(kThreads8);
   if (a.dq)
-    k_down_rep<true><<<gd, bd, kDnDqLds, s>>>(a);
+    k_down_rep<true, false><<<gd, bd, kDnDqLds, s>>>(a);
+  else if (a.st_dn_rows)
+    k_down_rep<false, true><<<gd, bd, kDnRowsLds, s>>>(a);
   else
-    k_down_rep<false><<<gd, bd, kDnLds, s>>>(a);
+    k_down_rep<false, false><<<gd, bd, kDnLds, s>>>(a);
   if (a.st_dn_gx > 1) hipLaunchKernelGGL(k_fin_rep, dim3(a.H / 256), dim3(256), 0, s, a);
 }
 

@@ -1,0 +1,56 @@
+"""Decode over row-major gathered down weights at the edges of their tiling;
+equalities are exact."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _np(t):
+    return t.detach().cpu().contiguous().numpy()
+
+
+def _gather(orc, L, blocks):
+    gp, ga = orc.gather_rows_blocks(_np(L.gate_packed), _np(L.gate_absmax), blocks, L.H, L.qbs)
+    upk, ua = orc.gather_rows_blocks(_np(L.up_packed), _np(L.up_absmax), blocks, L.H, L.qbs)
+    dp, da = orc.gather_down_columns(_np(L.down_packed), _np(L.down_absmax), blocks, L.H, L.I, L.qbs)
+    return gp, ga, upk, ua, dp, da
+
+
+@pytest.mark.parametrize("H,A,kk", [
+    (2048, 2, 1),
+    (2048, 48, 48),     # one wave's blocks cut over block groups
+    (4096, 300, 300),   # tiles of a wave ending in 1 to 3 blocks
+    (16384, 520, 515),  # more blocks than one workgroup's activations hold at one group: the last tile is short
+])
+def test_gathered_down_equals_slot_path(gpu, orc, H, A, kk):
+    """Row-major gathered blocks in any order, with entries left out (-1):
+    the bits of the slot-table decode over the same blocks in that order."""
+    from next_step_ai_amd.sparse_mlp import triton_fused_sparse_mlp_decode_4bit
+    from next_step_ai_amd.synth import make_synthetic_layer
+
+    print(f"gathered H={H} A={A} kk={kk}", flush=True)
+    I = 32 * ((A + 3) // 4 * 4)
+    L = make_synthetic_layer(H=H, I=I, R=16, seed=A + kk, device=gpu)
+    gp, ga, upk, ua, dp, da = _gather(orc, L, np.arange(A, dtype=np.int64))
+    rng = np.random.default_rng(kk)
+    idx = rng.permutation(A)[:kk].astype(np.int32)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu).reshape(-1)  # noqa: E731
+    code = torch.tensor(orc.nf4_code(), device=gpu)
+
+    def fused(ids):
+        return triton_fused_sparse_mlp_decode_4bit(
+            L.x.reshape(1, H), t(ids).reshape(1, -1), torch.ones((1, A * 32), dtype=torch.float16, device=gpu),
+            gate_packed_weight=t(gp), gate_absmax=t(ga), gate_code=code, gate_input_dim=H, gate_quant_block_size=64,
+            gate_bias=None, up_packed_weight=t(upk), up_absmax=t(ua), up_code=code, up_input_dim=H,
+            up_quant_block_size=64, up_bias=None, down_packed_weight=t(dp), down_absmax=t(da), down_code=code,
+            down_out_features=H, down_in_features=A * 32, down_quant_block_size=32, down_bias=None,
+            block_size=32).reshape(-1)
+
+    assert torch.equal(fused(idx), L.slot_table().decode(L.x, t(idx)))
+    if kk > 2:
+        holes = idx.copy()
+        holes[1::3] = -1
+        kept = L.slot_table(resident_blocks=t(idx[[i for i in range(kk) if i % 3 != 1]]))
+        assert torch.equal(fused(holes), kept.decode(L.x, t(idx)))
