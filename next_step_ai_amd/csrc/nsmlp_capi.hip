@@ -748,7 +748,7 @@ int nsmlp_decode_layer_noalloc_f16(const nsmlp_router* router, const nsmlp_slot_
   a.out = (uint16_t*)out;
   a.residual = (const uint16_t*)residual;
   fill_decode_tiling(a);
-  if (a.st_gu_wgs <= 0 || !streaming_can_select(a.NB, k))
+  if (a.H % 2048 != 0 || a.st_gu_wgs <= 0 || !streaming_can_select(a.NB, k))
     return set_error(NSMLP_EINVAL,
                      "no-allocation decode covers the streaming kernels only: hidden size a multiple of 2048 up to "
                      "16384, num_blocks <= 4096, k <= 2048 (got H=%d, num_blocks=%d, k=%d)",

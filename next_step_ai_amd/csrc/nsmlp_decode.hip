@@ -5,9 +5,9 @@
 // one fp16 rounding of the output).  Deterministic: no float atomics, every
 // sum is taken in a fixed order.
 //
-// The streaming kernels for hidden sizes that are a multiple of 2048 live in
-// nsmlp_stream.hip.
-// Generic path (any hidden size that is a multiple of 256, any down layout):
+// The streaming kernels for hidden sizes up to 16384 live in nsmlp_stream.hip.
+// Generic path (larger hidden sizes, strides that differ between slots and
+// host copies, offsets past 31 bits; any down layout):
 // k_gate_up / k_down, the same arithmetic in two launches with a last-arriver
 // hand-off.
 #include "nsmlp_internal.h"

@@ -694,7 +694,7 @@ struct DecodeArgs {
   int* row_count;        // [H / rows_per_chunk]
   int* status;           // [1] device error flag
   int chunks;            // down row chunks
-  // streaming path (hidden size a multiple of 2048)
+  // streaming path (hidden size a multiple of 256 up to 16384)
   float* st_act;         // [k][32] silu(gate) * up of the selected blocks
   uint32_t* st_enc;      // [k] resolved block references
   int st_gu_wgs;         // gate/up workgroups (0: streaming path not used)
@@ -905,7 +905,7 @@ void launch_cache_record(float* counts, int NB, const int32_t* blocks, int rows,
 
 void launch_decode_gate_up(const DecodeArgs& a, hipStream_t s);
 void launch_decode_down(const DecodeArgs& a, hipStream_t s);
-// Streaming decode (hidden size a multiple of 2048): gate/up, down, final sum.
+// Streaming decode (hidden size a multiple of 256 up to 16384): gate/up, down, final sum.
 // Sets the st_* tiling fields for a device with `cus` compute units; false
 // (and st_gu_wgs = 0) when the streaming kernels do not apply.
 bool plan_streaming(DecodeArgs& a, int cus);

@@ -1,5 +1,5 @@
-// Streaming sparse-MLP decode for hidden sizes that are a multiple of 2048
-// (one wave covers a 2048-column split: 64 lanes x 32 columns).
+// Streaming sparse-MLP decode for hidden sizes that are a multiple of 256, up
+// to 16384 (one wave covers a 2048-column split: 64 lanes x 32 columns).
 //
 //   k_gu_rep    gate/up.  An 8-wave workgroup works in rounds; in a round every
 //               wave decodes one item: gate rows 2p, 2p+1 and up rows 2p, 2p+1
@@ -99,12 +99,14 @@ struct GuStage {
   uint32_t qa[2];  // double-quantised: u8 codes of gate rows 2p | 2p+1 << 8, same for up
 };
 
-// Issue the loads of one item (block reference enc, row pair p).  ca: this
-// lane's absmax entry inside a row (its columns / qbs); cb: its byte offset
-// inside a packed row.
-template <bool DQ>
-__device__ __forceinline__ void gu_issue(const DecodeArgs& a, uint32_t enc, int p, uint32_t cb, uint32_t ca,
-                                         GuStage& st) {
+// Issue the loads of one item (block reference enc, block id bid, row pair p).
+// ca: this lane's absmax entry inside a row (its columns / qbs); cb: its byte
+// offset inside a packed row.  RAG: a row does not fill its splits, and the
+// lanes past its end (colok false) read zeros; the absmax2 are read per lane,
+// as a split may straddle second-level blocks.
+template <bool DQ, bool RAG>
+__device__ __forceinline__ void gu_issue(const DecodeArgs& a, uint32_t enc, uint32_t bid, int p, bool colok, uint32_t cb,
+                                         uint32_t ca, GuStage& st) {
   const bool bad = (enc & kBad) != 0;
   const bool dev = (enc & kHostBit) == 0;
   const long long q = bad ? 0 : (long long)(enc & (kHostBit - 1));
@@ -113,6 +115,7 @@ __device__ __forceinline__ void gu_issue(const DecodeArgs& a, uint32_t enc, int 
   const rsrc_t ru = make_rsrc((dev ? a.up.packed : a.host_up.packed) + q * a.up.blk_stride, nb);
   const uint32_t rs = (uint32_t)a.gate.row_stride, ars = (uint32_t)a.gate.abs_row_stride;
   const uint32_t s0 = (uint32_t)(2 * p) * rs;
+  if constexpr (RAG) cb = colok ? cb : kOffNone;
   st.w[0] = buf_ld16(rg, cb, s0);
   st.w[1] = buf_ld16(rg, cb, s0 + rs);
   st.w[2] = buf_ld16(ru, cb, s0);
@@ -121,13 +124,23 @@ __device__ __forceinline__ void gu_issue(const DecodeArgs& a, uint32_t enc, int 
     // codes of rows 2p and 2p+1 at entry ca: one 16-bit read per projection
     const rsrc_t rgq = make_rsrc((dev ? a.gate.qabsmax : a.host_gate.qabsmax) + q * a.gate.abs_blk_stride, na);
     const rsrc_t ruq = make_rsrc((dev ? a.up.qabsmax : a.host_up.qabsmax) + q * a.up.abs_blk_stride, na);
-    const uint32_t qo = ((uint32_t)p * ars + ca) * 2u;
+    uint32_t qo = ((uint32_t)p * ars + ca) * 2u;
+    if constexpr (RAG) {
+      qo = colok ? qo : kOffNone;
+      const rsrc_t rg2 = make_rsrc(a.gate.absmax2, a.st_gu_a2bytes), ru2 = make_rsrc(a.up.absmax2, a.st_gu_a2bytes);
+      const uint32_t f = (32u * bid + 2u * (uint32_t)p) * ars + ca;
+      const uint32_t o0 = colok ? (f >> a.dq_shift) * 4u : kOffNone, o1 = colok ? ((f + ars) >> a.dq_shift) * 4u : kOffNone;
+      st.am[0] = buf_ldfc(rg2, o0, 0);
+      st.am[1] = buf_ldfc(rg2, o1, 0);
+      st.am[2] = buf_ldfc(ru2, o0, 0);
+      st.am[3] = buf_ldfc(ru2, o1, 0);
+    }
     st.qa[0] = buf_ldu16(rgq, qo, 0);
     st.qa[1] = buf_ldu16(ruq, qo, 0);
   } else {
     const rsrc_t rga = make_rsrc((dev ? a.gate.absmax : a.host_gate.absmax) + q * a.gate.abs_blk_stride, na);
     const rsrc_t rua = make_rsrc((dev ? a.up.absmax : a.host_up.absmax) + q * a.up.abs_blk_stride, na);
-    const uint32_t ars4 = ars * 4u, as0 = (uint32_t)(2 * p) * ars4, ca4 = ca * 4u;
+    const uint32_t ars4 = ars * 4u, as0 = (uint32_t)(2 * p) * ars4, ca4 = RAG && !colok ? kOffNone : ca * 4u;
     st.am[0] = buf_ldf(rga, ca4, as0);
     st.am[1] = buf_ldf(rga, ca4, as0 + ars4);
     st.am[2] = buf_ldf(rua, ca4, as0);
@@ -192,7 +205,7 @@ __device__ __forceinline__ void pin_gu_first(DecodeArgs& a, int& nwg) {
   auto gc2 = gptr(a.gate.code2), uc2 = gptr(a.up.code2);
   asm volatile(""
                : "+s"(nwg), "+s"(x), "+s"(sel), "+s"(sel_scores), "+s"(code), "+s"(code_up), "+s"(gc2), "+s"(uc2),
-                 "+s"(a.splits), "+s"(a.NB), "+s"(a.k), "+s"(a.st_gu_rounds));
+                 "+s"(a.splits), "+s"(a.NB), "+s"(a.k), "+s"(a.H), "+s"(a.st_gu_rounds));
   a.x = (const uint16_t*)x;
   a.sel = (const int32_t*)sel;
   a.sel_scores = (const uint16_t*)sel_scores;
@@ -249,14 +262,18 @@ __device__ __forceinline__ void pin_gu_rest(DecodeArgs& a) {
   a.gate.absmax2 = (const float*)g2;
   a.up.absmax2 = (const float*)u2;
   auto served = gptr(a.served);
-  asm volatile("" : "+s"(served));
+  asm volatile("" : "+s"(served), "+s"(a.st_gu_a2bytes));
   a.served = (uint32_t*)served;
 }
 
 // SKPT > 0: the workgroup first selects the top k of a.sel_scores itself (SKPT
 // scores per thread; ascending ids, ties to the lower id), so the selection
 // needs no launch of its own; workgroup 0 also writes the ids to a.sel_out.
-template <bool AFFINE, int SKPT, bool DQ>
+// RAG: any number of splits up to 8, the last one partly past the row's end;
+// the waves past the last whole item of a round stay idle.  At hidden 5120
+// (2.5 splits, two waves idle), 61 blocks, a layer takes 27.4 us, against 54
+// in the two-launch kernels with a selection of its own (k_gate_up, k_down).
+template <bool AFFINE, int SKPT, bool DQ, bool RAG>
 __global__ void __launch_bounds__(kThreads8, 2) k_gu_rep(DecodeArgs args) {
   DecodeArgs a = args;
   int nwg;
@@ -266,21 +283,22 @@ __global__ void __launch_bounds__(kThreads8, 2) k_gu_rep(DecodeArgs args) {
   int* okl = reinterpret_cast<int*>(lds + kGuOkWord);
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform per wave
-  const int S = a.splits;                                     // 1, 2, 4 or 8
-  const int sh = __builtin_ctz((unsigned)S);  // S is a power of two
-  const int NS = kWaves >> sh;
-  const int s = wave & (S - 1), q = wave >> sh;
+  const int S = a.splits;                                     // 1, 2, 4 or 8 (RAG: 1..8)
+  const int sh = __builtin_ctz((unsigned)S);
+  const int NS = RAG ? kWaves / S : kWaves >> sh;
+  const int s = RAG ? wave % S : wave & (S - 1), q = RAG ? wave / S : wave >> sh;
   const int R = a.st_gu_rounds;
   const int wg = (int)blockIdx.x;
   const int n_items = 16 * a.k;
   const uint32_t col = (uint32_t)(s * kSplit + lane * 32);
+  const bool colok = !RAG || (int)col < a.H;
   const uint32_t cb = col >> 1, ca = col >> a.qbs_shift;
   const float* c2 = reinterpret_cast<const float*>(lds + kGuCode2Word);
 
   // Independent loads first: the block id of each lane's item (lane i:
   // round i), the code book and the token split.
   const int id0 = (lane * nwg + wg) * NS + q;
-  const bool own = lane < R && id0 < n_items;
+  const bool own = lane < R && id0 < n_items && (!RAG || q < NS);
   const int jb = own ? id0 >> 4 : 0;
   int b_id = 0;
   constexpr int kKeys = SKPT > 0 ? SKPT : 1;
@@ -301,10 +319,11 @@ __global__ void __launch_bounds__(kThreads8, 2) k_gu_rep(DecodeArgs args) {
   if constexpr (DQ) c2v = (tid < 256 ? a.gate.code2 : a.up.code2)[tid & 255];
   uint32_t xp[16];
   {
-    const uint4* xv = reinterpret_cast<const uint4*>(a.x + col);
+    const uint4* xv = reinterpret_cast<const uint4*>(a.x + (colok ? col : 0u));
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const uint4 t = xv[v];
+      uint4 t = xv[v];
+      if (!colok) t = make_uint4(0u, 0u, 0u, 0u);
       xp[4 * v] = t.x;
       xp[4 * v + 1] = t.y;
       xp[4 * v + 2] = t.z;
@@ -354,7 +373,7 @@ __global__ void __launch_bounds__(kThreads8, 2) k_gu_rep(DecodeArgs args) {
   // this wave's split (a 2048-column split never straddles a second-level
   // block), read once here instead of in the weight stream
   float a2_v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  if constexpr (DQ) {
+  if constexpr (DQ && !RAG) {
     const uint32_t ars = (uint32_t)a.gate.abs_row_stride;
     const uint32_t f0 = (32u * bid_v + 2u * (uint32_t)(id0 & 15)) * ars + (uint32_t)(s * kSplit >> a.qbs_shift);
     const uint32_t g0 = f0 >> a.dq_shift, g1 = (f0 + ars) >> a.dq_shift;
@@ -370,7 +389,8 @@ __global__ void __launch_bounds__(kThreads8, 2) k_gu_rep(DecodeArgs args) {
   GuStage st[kGuStages];
 #pragma unroll
   for (int i = 0; i < kGuStages; ++i)
-    gu_issue<DQ>(a, i < R ? lane_value(enc_v, i) : kBad, ((i * nwg + wg) * NS + q) & 15, cb, ca, st[i]);
+    gu_issue<DQ, RAG>(a, i < R ? lane_value(enc_v, i) : kBad, RAG ? lane_value(bid_v, i) : 0u,
+                      ((i * nwg + wg) * NS + q) & 15, colok, cb, ca, st[i]);
   sched_fence();
   // block-source counts (behind the stages: nothing waits for them early),
   // one per selected block: its row pair 0 at split 0
@@ -405,7 +425,7 @@ __global__ void __launch_bounds__(kThreads8, 2) k_gu_rep(DecodeArgs args) {
         float a2[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         if constexpr (DQ) {
 #pragma unroll
-          for (int m = 0; m < 4; ++m) a2[m] = __uint_as_float(lane_value(__float_as_uint(a2_v[m]), r));
+          for (int m = 0; m < 4; ++m) a2[m] = RAG ? st[i].am[m] : __uint_as_float(lane_value(__float_as_uint(a2_v[m]), r));
         }
         acc[0] = rep_dot32(st[i].w[0], xp, adg) * gu_absmax<DQ>(a, st[i], c2, 0, a2[0]);
         acc[1] = rep_dot32(st[i].w[1], xp, adg) * gu_absmax<DQ>(a, st[i], c2, 1, a2[1]);
@@ -414,12 +434,13 @@ __global__ void __launch_bounds__(kThreads8, 2) k_gu_rep(DecodeArgs args) {
       }
       const int rn = r + kGuStages;
       const int rl = rn < R && rn < kMaxItems ? rn : 0;
-      gu_issue<DQ>(a, rn < R ? lane_value(enc_v, rl) : kBad, ((rn * nwg + wg) * NS + q) & 15, cb, ca, st[i]);
+      gu_issue<DQ, RAG>(a, rn < R ? lane_value(enc_v, rl) : kBad, RAG ? lane_value(bid_v, rl) : 0u,
+                        ((rn * nwg + wg) * NS + q) & 15, colok, cb, ca, st[i]);
       if (live) {
         const float v = reduce4(acc, lane);
         if ((lane & 15) == 0) comb[r * (kWaves * 4) + wave * 4 + (lane >> 4)] = v;
         if constexpr (AFFINE) {
-          if (s == 0 && lane == 0) okl[r * kWaves + q] = !(lane_value(enc_v, r) & kBad);
+          if (s == 0 && lane == 0 && (!RAG || q < NS)) okl[r * kWaves + q] = !(lane_value(enc_v, r) & kBad);
         }
       }
     }
@@ -563,11 +584,12 @@ __global__ void __launch_bounds__(kThreads8, 2) k_down_rep(DecodeArgs args) {
   const int GX = a.st_dn_gx, per = a.st_dn_per;
   // XCD-aware mapping: workgroups go to the 8 XCDs round-robin (b % 8);
   // chunks 2m and 2m+1 share the 128-byte lines of the absmax codes, so
-  // both are given to workgroups of one XCD (one L2).  The grid size
-  // (H / 64) GX is a multiple of 16 (H a multiple of 2048).
+  // both are given to workgroups of one XCD (one L2).  The last (H / 64) GX
+  // % 16 workgroups (none where H is a multiple of 1024) pair up in order.
   const uint32_t xcd = blockIdx.x & 7u, sidx = blockIdx.x >> 3;
-  const uint32_t m = xcd + 8u * (sidx >> 1);
-  const int gx = (int)(m % (uint32_t)GX), c = 2 * (int)(m / (uint32_t)GX) + (int)(sidx & 1u);
+  const bool whole = (blockIdx.x | 15u) < gridDim.x;
+  const uint32_t m = whole ? xcd + 8u * (sidx >> 1) : blockIdx.x >> 1;
+  const int gx = (int)(m % (uint32_t)GX), c = 2 * (int)(m / (uint32_t)GX) + (int)((whole ? sidx : blockIdx.x) & 1u);
   const int nbw_all = (a.k + GX - 1) / GX;
   const int jb0 = gx * nbw_all;
   const int nbw = max(0, min(a.k - jb0, nbw_all));  // blocks of this workgroup
@@ -948,7 +970,7 @@ int device_cus() {
 
 bool plan_streaming(DecodeArgs& a, int cus) {
   a.st_gu_wgs = 0;
-  if (a.H % kSplit != 0 || a.H / kSplit > kWaves || cus <= 0) return false;
+  if (a.H % 256 != 0 || a.H > kSplit * kWaves || cus <= 0) return false;
   if (a.n_slots >= (1 << 30)) return false;
   // one set of strides for HBM slots and host copies; 32-bit extents
   if (a.gate.row_stride != a.up.row_stride || a.gate.abs_row_stride != a.up.abs_row_stride) return false;
@@ -976,7 +998,7 @@ bool plan_streaming(DecodeArgs& a, int cus) {
     a.st_gu_a2bytes = (int)(n2 * 4);
     a.st_dn_a2n = (int)a2n;
   }
-  const int S = a.H / kSplit;
+  const int S = (a.H + kSplit - 1) / kSplit;
   const int NS = kWaves / S;
   // gate/up: rounds of NS items per workgroup, balanced over the workgroups
   const long long items = 16LL * a.k;
@@ -1017,23 +1039,27 @@ bool streaming_can_select(int NB, int k) { return NB >= 1 && NB <= kSelMaxNB && 
 
 void launch_decode_streaming(const DecodeArgs& a, hipStream_t s) {
   using GuFn = void (*)(DecodeArgs);
-  // [dq][affine][0: given ids, 1: top-k of 4 scores per thread, 2: of 8]
-  static const GuFn gu_fns[2][2][3] = {
-      {{k_gu_rep<false, 0, false>, k_gu_rep<false, 4, false>, k_gu_rep<false, 8, false>},
-       {k_gu_rep<true, 0, false>, k_gu_rep<true, 4, false>, k_gu_rep<true, 8, false>}},
-      {{k_gu_rep<false, 0, true>, k_gu_rep<false, 4, true>, k_gu_rep<false, 8, true>},
-       {k_gu_rep<true, 0, true>, k_gu_rep<true, 4, true>, k_gu_rep<true, 8, true>}}};
+  // [ragged][dq][affine][0: given ids, 1: top-k of 4 scores per thread, 2: of 8]
+#define NSMLP_GU(RAG, DQ, AFF) {k_gu_rep<AFF, 0, DQ, RAG>, k_gu_rep<AFF, 4, DQ, RAG>, k_gu_rep<AFF, 8, DQ, RAG>}
+  static const GuFn gu_fns[2][2][2][3] = {
+      {{NSMLP_GU(false, false, false), NSMLP_GU(false, false, true)},
+       {NSMLP_GU(false, true, false), NSMLP_GU(false, true, true)}},
+      {{NSMLP_GU(true, false, false), NSMLP_GU(true, false, true)},
+       {NSMLP_GU(true, true, false), NSMLP_GU(true, true, true)}}};
+#undef NSMLP_GU
   std::call_once(g_attr_once, [] {
-    for (int d = 0; d < 2; ++d)
-      for (int f = 0; f < 2; ++f)
-        for (int m = 0; m < 3; ++m) set_lds_limit(gu_fns[d][f][m], m ? kGuSelLds : (d ? kGuDqLds : kGuLds));
+    for (int g = 0; g < 2; ++g)
+      for (int d = 0; d < 2; ++d)
+        for (int f = 0; f < 2; ++f)
+          for (int m = 0; m < 3; ++m) set_lds_limit(gu_fns[g][d][f][m], m ? kGuSelLds : (d ? kGuDqLds : kGuLds));
     set_lds_limit(k_down_rep<false, false>, kDnLds);
     set_lds_limit(k_down_rep<false, true>, kDnRowsLds);
     set_lds_limit(k_down_rep<true, false>, kDnDqLds);
   });
   const bool affine = a.gate_bias != nullptr || a.up_bias != nullptr || a.mask != nullptr;
   const int mode = a.sel_scores == nullptr ? 0 : (a.NB <= 4 * kThreads8 ? 1 : 2);
-  const GuFn gu = gu_fns[a.dq ? 1 : 0][affine ? 1 : 0][mode];
+  const bool pow2 = a.H % kSplit == 0 && (a.splits & (a.splits - 1)) == 0;
+  const GuFn gu = gu_fns[pow2 ? 0 : 1][a.dq ? 1 : 0][affine ? 1 : 0][mode];
   const size_t gu_lds = mode ? (size_t)kGuSelWord * 4 + (size_t)a.k * sizeof(int32_t) : (a.dq ? kGuDqLds : kGuLds);
   gu<<<dim3(a.st_gu_wgs), dim3(kThreads8), gu_lds, s>>>(a);
   const dim3 gd((a.H / kWave) * a.st_dn_gx), bd(kThreads8);
