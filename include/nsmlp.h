@@ -407,7 +407,8 @@ typedef struct nsmlp_nf4_matrix {
  *   out[t][o] = sum_c W[o][c] x[t][c],  t < rows
  * x [rows][in] fp16 (16-byte aligned), out [rows][out] fp16, out_f32
  * [rows][out] (nullable) the same sums before the fp16 rounding.  One pass
- * over the weight per two rows.  in_features > 16384: use
+ * over the weight per row or two; with three rows or more, in a multiple of
+ * 128 and qbs >= 64, per 32 rows.  in_features > 16384: use
  * nsmlp_input_linear_nf4_f16 with every block active. */
 int nsmlp_dense_linear_nf4_f16(const nsmlp_nf4_matrix* w, const void* x, int rows, void* out, float* out_f32,
                                void* stream);

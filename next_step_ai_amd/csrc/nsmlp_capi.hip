@@ -1191,13 +1191,17 @@ int nsmlp_dense_linear_nf4_f16(const nsmlp_nf4_matrix* w, const void* x, int row
   }
   a.code = w->code;
   const int cus = device_cus();
-  for (int t = 0; t < rows; t += 2) {
-    const int nt = rows - t >= 2 ? 2 : 1;
-    if (!plan_rows(a, nt, cus)) return set_error(NSMLP_EINVAL, "dense linear geometry not supported");
+  for (int t = 0, nt; t < rows; t += nt) {
+    const bool few = few_tokens_rows_fit(a, rows - t);
+    nt = rows - t >= 2 ? 2 : 1;
+    if (!few && !plan_rows(a, nt, cus)) return set_error(NSMLP_EINVAL, "dense linear geometry not supported");
     a.x = (const uint16_t*)x + (long long)t * in;
     a.y = (uint16_t*)out + (long long)t * O;
     a.out_f32 = out_f32 ? out_f32 + (long long)t * O : nullptr;
-    launch_rows(a, nt, (hipStream_t)stream);
+    if (few)
+      nt = launch_few_tokens_rows(a, rows - t, (hipStream_t)stream);
+    else
+      launch_rows(a, nt, (hipStream_t)stream);
   }
   return check_launch("dense linear");
 }

@@ -1,6 +1,6 @@
 // Few-token products over NF4 rows on v_mfma_f32_16x16x32_f16: the sparse MLP
 // of up to 32 tokens over the union of their blocks (a short prefill chunk, a
-// batch of sequences decoded together).
+// batch of sequences decoded together), and an LM head of three rows or more.
 //
 // With few tokens the product is bound by the weight stream, as a decode is:
 // every union block is read once for all tokens, and a 16-token MFMA tile
@@ -37,6 +37,7 @@
 // registers) leave the lookups' and MFMAs' latency partly open (without the
 // weight loads gate/up still takes 133 us); the loads are temporal, as a row's
 // 128-byte line serves two chunks (172 -> 158 us against nontemporal ones).
+#include <cstring>
 #include <mutex>
 #include <utility>
 
@@ -183,7 +184,11 @@ struct FtGeo {
   static_assert(kLds <= 160 * 1024, "LDS");
 };
 
-template <bool DQ, int NT, int NCH>
+//
+// HEAD: the rows of one dense matrix instead (the LM head: d.gate and d.up are
+// both the matrix, p.rows its rows, a pair 32 of them), their sums rounded to
+// fp16 and, with p.out_f32, also written before that.
+template <bool DQ, int NT, int NCH, bool HEAD>
 __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
   using G = FtGeo<NT, NCH>;
   constexpr int SU = G::SU, PD = G::PD, RB = G::RB, NH = G::NH;
@@ -198,10 +203,10 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
   const int H = d.H, M = p.M, p_a2 = p.gu_a2bytes;
   const int CW = p.gu_cw, RW = kFtWaves / CW, CGS = p.gu_cgs, chunks = H >> 7;
   const int cw = wave & (CW - 1), rw = wave / CW;
-  const int nu = p.nu[0];
   // pairs: (union block, 16-row half), each a gate and an up tile
-  const int p_lo = (int)(blockIdx.x * (2u * (unsigned)nu) / gridDim.x);
-  const int p_hi = (int)((blockIdx.x + 1) * (2u * (unsigned)nu) / gridDim.x);
+  const unsigned pairs = HEAD ? (unsigned)(p.rows + 31) / 32 : 2u * (unsigned)p.nu[0];
+  const int p_lo = (int)(blockIdx.x * pairs / gridDim.x);
+  const int p_hi = (int)((blockIdx.x + 1) * pairs / gridDim.x);
   {
     LutCodes codes;
     lut_codes_load(d.code, d.code_up, tid, codes);
@@ -225,14 +230,26 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
     uint32_t qa[NH];
     float am[NH];
   };
-  for (int pb = p_lo; pb < p_hi; pb += G::kSlots / 2) {
-    const int np = min(p_hi - pb, G::kSlots / 2), ntl = 2 * np;
+  // equal batches of at most kSlots tiles
+  const int batches = (p_hi - p_lo + G::kSlots / 2 - 1) / (G::kSlots / 2);
+  const int step = HEAD ? (p_hi - p_lo + batches - 1) / max(batches, 1) : G::kSlots / 2;
+  for (int pb = p_lo; pb < p_hi; pb += step) {
+    const int np = min(p_hi - pb, step), ntl = 2 * np;
     const int R = (ntl + RW - 1) / RW, VT = R * CGS;
     // lane t: tile t's packed rows and its block's absmax (addresses), the
     // flat index of its first absmax; bit 31 of that: the block is unavailable
     uint64_t tw = 0, ta = 0;
     uint32_t tf = 0x80000000u;
-    if (lane < ntl) {
+    if (HEAD && lane < ntl) {
+      const int r0 = 32 * pb + 16 * lane;
+      if (r0 < p.rows) {
+        tw = reinterpret_cast<uint64_t>(d.gate.packed + (long long)r0 * rs);
+        ta = DQ ? reinterpret_cast<uint64_t>(d.gate.qabsmax + (long long)r0 * A)
+                : reinterpret_cast<uint64_t>(d.gate.absmax + (long long)r0 * A);
+        tf = (uint32_t)r0 * A;
+      }
+    }
+    if (!HEAD && lane < ntl) {
       const int pi = pb + (lane >> 1), h16 = (pi & 1) * 16;
       const bool up = (lane & 1) != 0;
       const BlockRef br = resolve_id(d, p.ublk[pi >> 1]);
@@ -255,7 +272,8 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
       const uint32_t f = ft_lane(tf, l);
       const bool ok = live && (int)f >= 0;
       const int chb = (icg * CW + cw) * NCH;
-      const rsrc_t rp = make_rsrc(reinterpret_cast<const void*>(ft_lane64(tw, l)), ok ? 16 * (int)rs : 0);
+      const int nr = !ok ? 0 : HEAD ? min(p.rows - 32 * pb - 16 * l, 16) : 16;  // the tile's rows
+      const rsrc_t rp = make_rsrc(reinterpret_cast<const void*>(ft_lane64(tw, l)), nr * (int)rs);
       // temporal: a row's 128-byte line serves two chunks.  Columns past the
       // last chunk read the next row (or zeros past the tile): their tokens
       // are zero
@@ -263,14 +281,14 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
       constexpr int c0 = U == 0 ? 0 : SU, c1 = U == 0 ? SU : NCH;
 #pragma unroll
       for (int c = c0; c < c1; ++c) st.w[c - c0] = buf_ld16c(rp, voff + 64u * (uint32_t)c, 0);
-      const rsrc_t ra = make_rsrc(reinterpret_cast<const void*>(ft_lane64(ta, l)), ok ? (int)(16u * A * (DQ ? 1u : 4u)) : 0);
+      const rsrc_t ra = make_rsrc(reinterpret_cast<const void*>(ft_lane64(ta, l)), nr * (int)(A * (DQ ? 1u : 4u)));
       const rsrc_t r2 = make_rsrc(reinterpret_cast<const void*>(pick((t & 1) != 0, s_u, s_g)), ok ? p_a2 : 0);
 #pragma unroll
       for (int i = 0; i < (2 * (c1 - c0) + 3) / 4; ++i) {
         const uint32_t e = (uint32_t)(128 * chb + 64 * (2 * c0 + 4 * i + g)) >> qsh;
         if constexpr (DQ) {
-          // codes of rows 2 i and 2 i + 1 are interleaved
-          st.qa[i] = buf_ldu8c(ra, (uint32_t)(j & 14) * A + 2u * e + (uint32_t)(j & 1), 0);
+          // a slot's codes of rows 2 i and 2 i + 1 are interleaved
+          st.qa[i] = buf_ldu8c(ra, HEAD ? (uint32_t)j * A + e : (uint32_t)(j & 14) * A + 2u * e + (uint32_t)(j & 1), 0);
           st.am[i] = buf_ldfc(r2, ((f + (uint32_t)j * A + e) >> dsh) * 4u, 0);
         } else {
           st.qa[i] = 0;
@@ -375,11 +393,18 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
               for (int n = 0; n < NT; ++n)
                 cc[o][s >> 1][n] = mfma16(x[c][s][n], b[s], (s & 1) ? cc[o][s >> 1][n] : float4_t{0.0f, 0.0f, 0.0f, 0.0f});
           };
+          auto weights = [&](auto cc_) {
+            constexpr int c = decltype(cc_)::value;
+            if constexpr (c < SU)
+              return st[2 * i].w[c];
+            else
+              return st[2 * i + 1].w[c - SU];
+          };
           auto chunk = [&](auto cc_) {
             constexpr int c = decltype(cc_)::value;
             if constexpr (G::kPipe) {
               if constexpr (c + 1 < NCH) {
-                lookup(bq[(c + 1) & 1], c + 1 < SU ? st[2 * i].w[c + 1] : st[2 * i + 1].w[c + 1 - SU]);
+                lookup(bq[(c + 1) & 1], weights(std::integral_constant<int, c + 1>{}));
               } else {
                 set_ad(tn);
                 lookup(bq[(c + 1) & 1], st[(2 * i + 2) % PD].w[0]);
@@ -400,7 +425,7 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
             } else {
               if constexpr (c == 0) set_ad(t);
               if constexpr (c == SU) resolve(ar, st[2 * i + 1], SU, NCH - SU);
-              lookup(bq[0], c < SU ? st[2 * i].w[c] : st[2 * i + 1].w[c - SU]);
+              lookup(bq[0], weights(cc_));
               products(cc_, bq[0]);
               mfma_drain();
               scale(cc_);
@@ -439,6 +464,19 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
       }
     }
     lds_barrier();
+    if constexpr (HEAD) {
+      const int nr = min(16 * ntl, p.rows - 32 * pb);
+      for (int t = wave; t < M; t += kFtWaves)
+        for (int r = lane; r < nr; r += kWave) {
+          const float y = reinterpret_cast<const float*>(
+              slots + (r >> 4) * NT * 64)[((t >> 4) * 64 + ((t >> 2) & 3) * 16 + (r & 15)) * 4 + (t & 3)];
+          const long long o = (long long)t * p.rows + 32 * pb + r;
+          p.out[o] = f2h(y);
+          if (p.out_f32 != nullptr) p.out_f32[o] = y;
+        }
+      lds_barrier();
+      continue;
+    }
     // act of (pair, token, row): element e of lane 16 g + j of token tile n is
     // token 16 n + 4 g + e, row j
     for (int i = tid; i < np * NT * 256; i += kFtThreads) {
@@ -688,20 +726,21 @@ struct FtKernel {
   FtFn fn;
   size_t lds;
 };
-template <bool DQ, int NT, int NCH>
+template <bool DQ, int NT, int NCH, bool HEAD>
 constexpr FtKernel ft_gu() {
-  return FtKernel{k_ft_gu<DQ, NT, NCH>, FtGeo<NT, NCH>::kLds};
+  return FtKernel{k_ft_gu<DQ, NT, NCH, HEAD>, FtGeo<NT, NCH>::kLds};
 }
 template <bool DQ, bool HOST, int NT>
 constexpr FtKernel ft_down() {
   return FtKernel{k_ft_down<DQ, HOST, NT>, FdGeo<NT>::kLds};
 }
-// [dq][one token tile of 4, 5, 6, 8 chunks, two of 3, 4]
-const FtKernel kFtGu[2][6] = {
-    {ft_gu<false, 1, 4>(), ft_gu<false, 1, 5>(), ft_gu<false, 1, 6>(), ft_gu<false, 1, 8>(), ft_gu<false, 2, 3>(),
-     ft_gu<false, 2, 4>()},
-    {ft_gu<true, 1, 4>(), ft_gu<true, 1, 5>(), ft_gu<true, 1, 6>(), ft_gu<true, 1, 8>(), ft_gu<true, 2, 3>(),
-     ft_gu<true, 2, 4>()}};
+// [head][dq][one token tile of 4, 5, 6, 8 chunks, two of 3, 4]
+#define NSMLP_FT_GU(HEAD, DQ) \
+  {ft_gu<DQ, 1, 4, HEAD>(), ft_gu<DQ, 1, 5, HEAD>(), ft_gu<DQ, 1, 6, HEAD>(), \
+   ft_gu<DQ, 1, 8, HEAD>(), ft_gu<DQ, 2, 3, HEAD>(), ft_gu<DQ, 2, 4, HEAD>()}
+const FtKernel kFtGu[2][2][6] = {{NSMLP_FT_GU(false, false), NSMLP_FT_GU(false, true)},
+                                 {NSMLP_FT_GU(true, false), NSMLP_FT_GU(true, true)}};
+#undef NSMLP_FT_GU
 constexpr int kFtGuChunks[6] = {4, 5, 6, 8, 3, 4};
 // [dq][host copies][token tiles - 1]
 const FtKernel kFtDown[2][2][2] = {{{ft_down<false, false, 1>(), ft_down<false, false, 2>()},
@@ -716,7 +755,8 @@ void ft_set_lds() {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k.fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)k.lds);
     };
     for (int q = 0; q < 2; ++q) {
-      for (const FtKernel& k : kFtGu[q]) set(k);
+      for (int f = 0; f < 2; ++f)
+        for (const FtKernel& k : kFtGu[f][q]) set(k);
       for (int h = 0; h < 2; ++h)
         for (const FtKernel& k : kFtDown[q][h]) set(k);
     }
@@ -798,10 +838,51 @@ void launch_few_tokens(const FewTokArgs& args, void* ws, hipStream_t s) {
   p.gu_a2bytes = p.dn_a2bytes = (int)(n2 * 4);
   k_ft_list<<<dim3(1), dim3(1024), 0, s>>>(p);
   ft_set_lds();
-  ft_launch(kFtGu[d.dq ? 1 : 0][gu], cus, p, s);
+  ft_launch(kFtGu[0][d.dq ? 1 : 0][gu], cus, p, s);
   ft_launch(kFtDown[d.dq ? 1 : 0][d.host_down.packed != nullptr ? 1 : 0][NT - 1], cus, p, s);
   const long long n = (long long)p.M * d.H;
   k_ft_fin<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>(p);
+}
+
+// The few-row LM head against the passes of one or two rows it replaces
+// (k_rows_rep), fp32 absmax, one call: hidden 4096, 128256 rows, 5 tokens
+// 225 -> 61.5 us (4.8 TB/s), 16 tokens 790 -> 65, 32 tokens 92; hidden 16384,
+// 5 tokens 847 -> 247 us.  One and two rows stay there: they give bit-equal
+// logits with each other, and one row is faster (183 us at hidden 16384).
+// MFMA chunks want whole 128 columns, and an absmax of whole 64-column halves.
+bool few_tokens_rows_fit(const RowsArgs& a, int rows) {
+  return rows > 2 && a.in % 128 == 0 && a.qbs_shift >= 6 && device_cus() >= 64;
+}
+
+int launch_few_tokens_rows(const RowsArgs& a, int rows, hipStream_t s) {
+  FewTokArgs p;
+  memset(&p, 0, sizeof(p));
+  DecodeArgs& d = p.d;
+  d.H = a.in;
+  d.qbs_shift = a.qbs_shift;
+  d.dq = a.dq;
+  d.dq_shift = a.dq_shift;
+  d.gate.packed = a.packed;
+  d.gate.row_stride = a.rs;
+  d.gate.absmax = a.absmax;
+  d.gate.qabsmax = a.qabsmax;
+  d.gate.abs_row_stride = a.ars;
+  d.gate.absmax2 = a.absmax2;
+  d.gate.code2 = a.code2;
+  d.gate.offset = a.offset;
+  d.up = d.gate;
+  d.code = d.code_up = a.code;
+  p.x = a.x;
+  p.M = rows < kFtMaxTok ? rows : kFtMaxTok;
+  p.rows = a.out;
+  p.out = a.y;
+  p.out_f32 = a.out_f32;
+  p.gu_a2bytes = a.a2_bytes;
+  p.NT = ft_token_tiles(p.M);
+  const int gu = ft_columns(a.in, p.NT, &p.gu_cw, &p.gu_cgs);
+  ft_set_lds();
+  ft_launch(kFtGu[1][a.dq ? 1 : 0][gu], device_cus(), p, s);
+  return p.M;
 }
 
 }  // namespace nsmlp

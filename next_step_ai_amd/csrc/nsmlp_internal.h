@@ -808,6 +808,9 @@ struct FewTokArgs {
   float* part;            // [groups][M][H] fp32
   int gu_cw, gu_cgs;      // gate/up column waves of a workgroup, column groups
   int gu_a2bytes, dn_a2bytes;
+  // the rows of one dense matrix
+  int rows;
+  float* out_f32;         // [M][rows] or NULL
 };
 bool few_tokens_shape(int H, int NB, int M);  // what the workspace sizes depend on
 bool few_tokens_fit(const DecodeArgs& d, int M);
@@ -876,6 +879,9 @@ struct RowsArgs {
 };
 bool plan_rows(RowsArgs& a, int nt, int cus);  // nt tokens per pass (1 or 2)
 void launch_rows(const RowsArgs& a, int nt, hipStream_t s);
+// Three rows or more: up to 32 a launch (returns how many).
+bool few_tokens_rows_fit(const RowsArgs& a, int rows);
+int launch_few_tokens_rows(const RowsArgs& a, int rows, hipStream_t s);
 
 // Hot-block cache maintenance (fixed-capacity promotion and calibration
 // counts) over a slot table with pinned host copies.

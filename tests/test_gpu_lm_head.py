@@ -171,3 +171,41 @@ def test_dense_linear_tiny_and_ragged_shapes(gpu, orc, V, H, qbs, rows):
     out, f32 = _run(gpu, x, torch.from_numpy(packed).to(gpu), torch.from_numpy(absmax).to(gpu), code, V, H, qbs)
     assert np.array_equal(_np(f32).astype(np.float64), ref)
     assert np.array_equal(_np(out).view(np.uint16), orc.f32_to_f16_bits(ref.astype(np.float32)))
+
+
+@pytest.mark.parametrize("V,H,qbs,rows", [
+    (5, 128, 64, 3),          # part of one tile, one chunk
+    (33, 256, 128, 16),       # a third tile of one row, a full token tile
+    (1001, 4096, 64, 17),     # eight column waves, second token tile
+    (515, 5120, 64, 34),      # five chunks a wave; 32 rows, then a pass of two
+    (300, 10368, 128, 9),     # 81 chunks over two column groups, the last one part
+    (517, 16384, 256, 32),    # four column groups
+    (131001, 128, 64, 20),    # two batches of tile sums a workgroup
+])
+def test_dense_linear_few_rows(gpu, orc, V, H, qbs, rows):
+    """Three rows or more (the few-token kernel): known answers bit-exact, a
+    double-quantised absmax gives the bits of the resolved one, random weights
+    within the bound, an infinity stays in its row."""
+    from next_step_ai_amd.nested_absmax import NestedAbsmax
+
+    print(f"lm head few rows V={V} H={H} rows={rows}", flush=True)
+    rng = np.random.default_rng(V + H + rows)
+    packed, absmax, x, _ = _known_case(rng, V, H, qbs, rows)
+    x = np.clip(x, -2, 2).astype(np.float16)
+    code = torch.tensor(orc.nf4_code(), device=gpu)
+    pk = torch.from_numpy(packed).to(gpu)
+    out, f32 = _run(gpu, x, pk, torch.from_numpy(absmax).to(gpu), code, V, H, qbs)
+    ref = orc.dense_linear_nf4(x.view(np.uint16), packed, absmax, V, H, qbs)
+    assert np.array_equal(_np(f32).astype(np.float64), ref)
+    assert np.array_equal(_np(out).view(np.uint16), orc.f32_to_f16_bits(ref.astype(np.float32)))
+    packed, absmax, x = _random_case(gpu, orc, rng, V, H, qbs, rows)
+    pk = torch.from_numpy(packed).to(gpu)
+    nested = NestedAbsmax.quantize(torch.from_numpy(absmax).to(gpu))
+    out_n, f32_n = _run(gpu, x, pk, nested, code, V, H, qbs)
+    out_r, f32_r = _run(gpu, x, pk, nested.resolve(), code, V, H, qbs)
+    assert torch.equal(f32_n, f32_r) and torch.equal(out_n, out_r)
+    _check_random(orc, x, packed, _np(nested.resolve()), V, H, qbs, out_r, f32_r)
+    x[1, 7] = np.inf
+    out_i, _ = _run(gpu, x, pk, nested, code, V, H, qbs, with_f32=False)
+    others = [r for r in range(rows) if r != 1]
+    assert torch.equal(out_i[others], out_n[others]) and not torch.isfinite(out_i[1]).any()
