@@ -77,56 +77,75 @@ __global__ void __launch_bounds__(kThreads) k_out_finish(LinearArgs a) {
 }
 
 // ------------------------------------------------------------ input linear
-constexpr int kInBatch = 16;
+// A workgroup takes 64 output rows of one token, a lane a row and a wave an
+// eighth of the active slots, 8 slots (16 packed bytes each) in flight; the
+// wave sums meet in LDS in wave order.  Bound by latency and the lookups: a
+// thread a row over all slots left most of the chip idle (96 workgroups, 64
+// slots one after the other: hidden 4096, 6 tokens x 64 blocks of 268, 56.5
+// us; now 22).  Workgroups of the same rows go to one XCD (out / 64 a
+// multiple of 8): its L2 serves the lines that the tokens share.
+constexpr int kInThreads = 512, kInWaves = kInThreads / kWave, kInBatch = 8;
 
-__global__ void __launch_bounds__(kThreads) k_in_linear(LinearArgs a) {
-  const int o = blockIdx.x * kThreads + threadIdx.x;
-  const int t = blockIdx.y;
-  const int tid = threadIdx.x;
+__global__ void __launch_bounds__(kInThreads) k_in_linear(LinearArgs a) {
   __shared__ float lut[16];
-  __shared__ float xs[kInBatch][32];
-  __shared__ int slots[kInBatch];
+  __shared__ __attribute__((aligned(16))) float xs[kInWaves][kInBatch][32];
+  __shared__ float sums[kInWaves][kWave];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int o = blockIdx.x * kWave + lane;
+  const int t = blockIdx.y;
   if (tid < 16) lut[tid] = a.code[tid];
+  __syncthreads();
   const bool live = o < a.out_dim;
   const long long row_bytes = a.in_dim / 2;
   const long long row_abs = a.in_dim / a.qbs;
-  float acc = 0.0f;
+  const uint8_t* wr = a.packed + (live ? o : 0) * row_bytes;
+  const float* ar = a.absmax + (live ? o : 0) * row_abs;
+  const uint16_t* xr = a.x + (long long)t * a.in_dim;
   // active block e / bm contributes its 32-column slot e % bm
-  const int n = a.kk * a.bm;
-  for (int ib = 0; ib < n; ib += kInBatch) {
-    __syncthreads();
-    if (tid < kInBatch) {
-      const int e = ib + tid;
-      const int blk = e < n ? a.active_idx[(long long)t * a.kk + e / a.bm] : -1;
-      const long long sl = (long long)blk * a.bm + e % a.bm;
-      slots[tid] = (blk >= 0 && sl * 32 < a.in_dim) ? (int)sl : -1;
-    }
-    __syncthreads();
-    for (int e = tid; e < kInBatch * 32; e += kThreads) {
-      int i = e / 32, c = e % 32;
-      int sl = slots[i];
-      xs[i][c] = sl >= 0 ? h2f(a.x[(long long)t * a.in_dim + (long long)sl * 32 + c]) : 0.0f;
-    }
-    __syncthreads();
+  const int n = a.kk * a.bm, per = (n + kInWaves - 1) / kInWaves;
+  const int e1 = min(n, (wave + 1) * per);
+  float acc = 0.0f;
+  for (int ib = wave * per; ib < e1; ib += kInBatch) {
+    // lane 8 i + c: slot i's columns 4 c .. 4 c + 3
+    const int e = ib + (lane >> 3);
+    const int blk = e < e1 ? a.active_idx[(long long)t * a.kk + e / a.bm] : -1;
+    const long long sl = (long long)blk * a.bm + e % a.bm;
+    const int slot = (blk >= 0 && sl * 32 < a.in_dim) ? (int)sl : -1;
     uint4 w[kInBatch];
     float am[kInBatch];
 #pragma unroll
     for (int i = 0; i < kInBatch; ++i) {
-      const int sl = slots[i];
+      const int si = __builtin_amdgcn_readlane(slot, 8 * i);
       w[i] = make_uint4(0, 0, 0, 0);
       am[i] = 0.0f;
-      if (sl >= 0 && live) {
-        w[i] = *reinterpret_cast<const uint4*>(a.packed + (long long)o * row_bytes + (long long)sl * 16);
-        am[i] = a.absmax[(long long)o * row_abs + ((long long)sl * 32) / a.qbs];
+      if (si >= 0 && live) {
+        w[i] = *reinterpret_cast<const uint4*>(wr + (long long)si * 16);
+        am[i] = ar[((long long)si * 32) / a.qbs];
       }
     }
+    const int c = (lane & 7) * 4;
+    float4 xv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (slot >= 0) {
+      const uint16_t* xp = xr + (long long)slot * 32 + c;
+      xv = make_float4(h2f(xp[0]), h2f(xp[1]), h2f(xp[2]), h2f(xp[3]));
+    }
+    // the wave's own stage: LDS operations of a wave are done in order
+    *reinterpret_cast<float4*>(&xs[wave][lane >> 3][c]) = xv;
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int i = 0; i < kInBatch; ++i)
-      if (slots[i] >= 0) acc += nf4_dot32_f32(w[i], xs[i], lut) * am[i];
+      if (__builtin_amdgcn_readlane(slot, 8 * i) >= 0) acc += nf4_dot32_f32(w[i], xs[wave][i], lut) * am[i];
+    __builtin_amdgcn_wave_barrier();
   }
-  if (live) {
-    if (a.bias != nullptr) acc += h2f(a.bias[o]);
-    a.out[(long long)t * a.out_dim + o] = f2h(acc);
+  sums[wave][lane] = acc;
+  __syncthreads();
+  if (wave == 0 && live) {
+    float y = 0.0f;
+#pragma unroll
+    for (int v = 0; v < kInWaves; ++v) y += sums[v][lane];
+    if (a.bias != nullptr) y += h2f(a.bias[o]);
+    a.out[(long long)t * a.out_dim + o] = f2h(y);
   }
 }
 
@@ -343,8 +362,8 @@ void launch_output_linear(const LinearArgs& a, hipStream_t s) {
 }
 
 void launch_input_linear(const LinearArgs& a, hipStream_t s) {
-  dim3 grid(grid_for(a.out_dim), a.rows);
-  hipLaunchKernelGGL(k_in_linear, grid, dim3(kThreads), 0, s, a);
+  dim3 grid((unsigned)((a.out_dim + kWave - 1) / kWave), a.rows);
+  hipLaunchKernelGGL(k_in_linear, grid, dim3(kInThreads), 0, s, a);
 }
 
 void launch_zero_u32(uint32_t* p, long long n, hipStream_t s) {
