@@ -354,6 +354,21 @@ int nsmlp_fused_decode_gathered_f16(const void* x, int H, const int32_t* active_
                                     const void* down_bias, int qbs, void* out, void* ws, size_t ws_bytes,
                                     void* stream);
 
+/* The same call for several rows (version >= 106): the gate and up output
+ * linears below in one pass, act = fp16(silu(gate) * up) at the active slots,
+ * and the input linear over act, with their roundings (fp16 gate, up and act).
+ * x [rows][H], active_idx [rows][kk], flat_mask [rows][A*32], down packed
+ * [out_features][A*32] NF4 with quant block down_qbs, out [rows][out_features].
+ */
+size_t nsmlp_fused_rows_workspace_bytes(int rows, int H, int kk, int A);
+int nsmlp_fused_rows_gathered_f16(const void* x, int rows, int H, const int32_t* active_idx, int kk, int A,
+                                  const void* flat_mask, const uint8_t* gate_packed, const float* gate_absmax,
+                                  const float* gate_code, const void* gate_bias, const uint8_t* up_packed,
+                                  const float* up_absmax, const float* up_code, const void* up_bias, int qbs,
+                                  const uint8_t* down_packed, const float* down_absmax, const float* down_code,
+                                  const void* down_bias, int down_qbs, int out_features, void* out, void* ws,
+                                  size_t ws_bytes, void* stream);
+
 /* Replaces TSM:1340-1375 (triton_sparse_output_linear_4bit) with row-major
  * NF4 semantics (the reference's Triton kernel indexes a transposed payload,
  * TSM:634-635; this computes what its callers pass, RT:4630-4660):

@@ -107,6 +107,9 @@ SIGNATURES: dict[str, tuple] = {
     "nsmlp_single_kernel_decode_f16": (I32, [P, P, P, P, P, P, P, P, P, P, P, P, I32, I32, I32, I32, P, SZ, P]),
     "nsmlp_fused_decode_workspace_bytes": (SZ, [I32, I32]),
     "nsmlp_fused_decode_gathered_f16": (I32, [P, I32, P, I32, I32, P, P, P, P, P, P, P, P, P, P, P, P, P, I32, P, P, SZ, P]),
+    "nsmlp_fused_rows_workspace_bytes": (SZ, [I32, I32, I32, I32]),
+    "nsmlp_fused_rows_gathered_f16": (I32, [P, I32, I32, P, I32, I32, P, P, P, P, P, P, P, P, P, I32, P, P, P, P, I32, I32,
+                                            P, P, SZ, P]),
     "nsmlp_output_linear_workspace_bytes": (SZ, [I32, I32, I32]),
     "nsmlp_output_linear_nf4_f16": (I32, [P, I32, I32, P, I32, I32, P, P, P, P, I32, P, I32, P, P, SZ, P]),
     "nsmlp_input_linear_nf4_f16": (I32, [P, I32, I32, P, I32, P, P, P, I32, I32, P, I32, P, P]),

@@ -565,7 +565,7 @@ extern "C" {
 
 const char* nsmlp_last_error(void) { return g_err; }
 
-int nsmlp_version(void) { return 105; }
+int nsmlp_version(void) { return 106; }
 
 int nsmlp_fault_inject(const char* spec) { return fault_set(spec); }
 
@@ -1067,6 +1067,60 @@ int nsmlp_fused_decode_gathered_f16(const void* x, int H, const int32_t* active_
   if (rc) return rc;
   fill_decode_tiling(a);
   return run_decode(a, (hipStream_t)stream);
+}
+
+size_t nsmlp_fused_rows_workspace_bytes(int rows, int H, int kk, int A) {
+  return nsmlp_output_linear_workspace_bytes(rows, 2 * kk, H) + align_up((size_t)rows * A * 64);
+}
+
+int nsmlp_fused_rows_gathered_f16(const void* x, int rows, int H, const int32_t* active_idx, int kk, int A,
+                                  const void* flat_mask, const uint8_t* gate_packed, const float* gate_absmax,
+                                  const float* gate_code, const void* gate_bias, const uint8_t* up_packed,
+                                  const float* up_absmax, const float* up_code, const void* up_bias, int qbs,
+                                  const uint8_t* down_packed, const float* down_absmax, const float* down_code,
+                                  const void* down_bias, int down_qbs, int out_features, void* out, void* ws,
+                                  size_t ws_bytes, void* stream) {
+  NSMLP_FAULT_POINT("output_linear_nf4_f16");
+  NSMLP_FAULT_POINT("silu_mul_f16");
+  if (rows <= 0 || kk <= 0 || A <= 0) return set_error(NSMLP_EINVAL, "rows, kk and A must be positive");
+  if (H <= 0 || H % 256 != 0) return set_error(NSMLP_EINVAL, "input_dim %d must be a multiple of 256", H);
+  if (qbs <= 0 || qbs % 32 != 0 || H % qbs != 0)
+    return set_error(NSMLP_EINVAL, "quant block size %d must be a multiple of 32 dividing %d", qbs, H);
+  if (!x || !active_idx || !gate_packed || !gate_absmax || !gate_code || !up_packed || !up_absmax || !up_code || !out)
+    return set_error(NSMLP_EINVAL, "NULL tensor argument");
+  if (!aligned16(gate_packed) || !aligned16(up_packed))
+    return set_error(NSMLP_EINVAL, "packed weight must be 16-byte aligned");
+  const size_t need = nsmlp_fused_rows_workspace_bytes(rows, H, kk, A);
+  if (ws == nullptr || ws_bytes < need)
+    return set_error(NSMLP_ENOSPC, "fused-rows workspace needs %zu bytes, got %zu", need, ws_bytes);
+  LinearArgs l;
+  memset(&l, 0, sizeof(l));
+  l.x = (const uint16_t*)x;
+  l.rows = rows;
+  l.in_dim = H;
+  l.active_idx = active_idx;
+  l.kk = kk;
+  l.A = A;
+  l.packed = gate_packed;
+  l.absmax = gate_absmax;
+  l.code = gate_code;
+  l.bias = (const uint16_t*)gate_bias;
+  l.packed_up = up_packed;
+  l.absmax_up = up_absmax;
+  l.code_up = up_code;
+  l.bias_up = (const uint16_t*)up_bias;
+  l.qbs = qbs;
+  l.mask = (const uint16_t*)flat_mask;
+  l.cs = choose_cs(H, rows * kk);
+  l.splits = H / l.cs;
+  uint16_t* act = (uint16_t*)((char*)ws + align_up(kCounterBytes));
+  l.out = act;
+  l.part = (float*)((char*)act + align_up((size_t)rows * A * 64));
+  launch_output_linear(l, (hipStream_t)stream);
+  const int rc = check_launch("fused rows gate/up");
+  if (rc) return rc;
+  return nsmlp_input_linear_nf4_f16(act, rows, A * 32, active_idx, kk, down_packed, down_absmax, down_code, down_qbs,
+                                    out_features, down_bias, 32, out, stream);
 }
 
 size_t nsmlp_output_linear_workspace_bytes(int rows, int kk, int in_dim) {

@@ -995,6 +995,13 @@ struct LinearArgs {
   uint16_t* out;
   int cs, splits;             // output linear column split
   float* part;                // [rows*kk][splits][32]
+  // a second projection of the same rows and slots (packed_up not null): its
+  // partial sums follow the first's, and out is fp16(silu(first) * second) at
+  // the active slots, nothing elsewhere
+  const uint8_t* packed_up;
+  const float* absmax_up;
+  const float* code_up;
+  const uint16_t* bias_up;
   int bm;                     // input linear: 32-column slots per active block
 };
 

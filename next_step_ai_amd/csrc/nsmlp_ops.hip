@@ -20,6 +20,10 @@ namespace {
 constexpr int kThreads = 256;
 
 // ----------------------------------------------------------- output linear
+// With a second projection (gate and up of the fused call of several rows) one
+// launch takes both and k_out_finish forms act where it adds their splits:
+// hidden 4096, 6 tokens x 64 blocks: 15.7 + 4.6 us, against 20.8 + 7.2 in a
+// launch per projection, 5 for two zero fills and 2.5 for silu * up.
 template <int LPR>
 __global__ void __launch_bounds__(kThreads) k_out_partial(LinearArgs a) {
   constexpr int kStep = kThreads / LPR;  // rows per pass
@@ -31,8 +35,12 @@ __global__ void __launch_bounds__(kThreads) k_out_partial(LinearArgs a) {
   const int slot = a.active_idx[task];
   if (slot < 0 || slot >= a.A) return;
   const int tid = threadIdx.x;
+  const bool up = blockIdx.z != 0;  // the second projection
+  const uint8_t* packed = up ? a.packed_up : a.packed;
+  const float* absmax = up ? a.absmax_up : a.absmax;
+  float* part = a.part + (up ? (long long)a.rows * a.kk * a.splits * 32 : 0);
   __shared__ float lut[16];
-  if (tid < 16) lut[tid] = a.code[tid];
+  if (tid < 16) lut[tid] = (up ? a.code_up : a.code)[tid];
   const int cc = tid % LPR;
   const int r0 = tid / LPR;
   const int col = s * a.cs + cc * 32;
@@ -43,8 +51,8 @@ __global__ void __launch_bounds__(kThreads) k_out_partial(LinearArgs a) {
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
     const long long r = (long long)slot * 32 + r0 + i * kStep;
-    w[i] = *reinterpret_cast<const uint4*>(a.packed + r * row_bytes + (col >> 1));
-    am[i] = a.absmax[r * row_abs + col / a.qbs];
+    w[i] = *reinterpret_cast<const uint4*>(packed + r * row_bytes + (col >> 1));
+    am[i] = absmax[r * row_abs + col / a.qbs];
   }
   float xf[32];
   const uint16_t* xr = a.x + (long long)t * a.in_dim + col;
@@ -56,7 +64,7 @@ __global__ void __launch_bounds__(kThreads) k_out_partial(LinearArgs a) {
     float acc = nf4_dot32_f32(w[i], xf, lut) * am[i];
 #pragma unroll
     for (int m = LPR / 2; m >= 1; m >>= 1) acc += __shfl_xor(acc, m, kWave);
-    if (cc == 0) a.part[((long long)task * a.splits + s) * 32 + r0 + i * kStep] = acc;
+    if (cc == 0) part[((long long)task * a.splits + s) * 32 + r0 + i * kStep] = acc;
   }
 }
 
@@ -67,12 +75,21 @@ __global__ void __launch_bounds__(kThreads) k_out_finish(LinearArgs a) {
   const int t = task / a.kk;
   const int slot = a.active_idx[task];
   if (slot < 0 || slot >= a.A) return;
-  float acc = 0.0f;
-  for (int s = 0; s < a.splits; ++s) acc += a.part[((long long)task * a.splits + s) * 32 + r];
   const long long n = (long long)slot * 32 + r;
-  if (a.bias != nullptr) acc += h2f(a.bias[n]);
-  uint16_t y = f2h(acc);
-  if (a.mask != nullptr) y = f2h(h2f(y) * h2f(a.mask[(long long)t * a.A * 32 + n]));
+  // the projection's fp16 value, then its mask
+  auto value = [&](const float* part, const uint16_t* bias) {
+    float acc = 0.0f;
+    for (int s = 0; s < a.splits; ++s) acc += part[((long long)task * a.splits + s) * 32 + r];
+    if (bias != nullptr) acc += h2f(bias[n]);
+    uint16_t y = f2h(acc);
+    if (a.mask != nullptr) y = f2h(h2f(y) * h2f(a.mask[(long long)t * a.A * 32 + n]));
+    return y;
+  };
+  uint16_t y = value(a.part, a.bias);
+  if (a.packed_up != nullptr) {
+    const uint16_t u = value(a.part + (long long)a.rows * a.kk * a.splits * 32, a.bias_up);
+    y = f2h(silu_mul(h2f(y), h2f(u)));
+  }
   a.out[(long long)t * a.A * 32 + n] = y;
 }
 
@@ -351,7 +368,7 @@ unsigned grid_for(long long n) { return (unsigned)((n + kThreads - 1) / kThreads
 }  // namespace
 
 void launch_output_linear(const LinearArgs& a, hipStream_t s) {
-  dim3 grid(a.splits, a.rows * a.kk);
+  dim3 grid(a.splits, a.rows * a.kk, a.packed_up != nullptr ? 2 : 1);
   switch (a.cs / 32) {
     case 8: hipLaunchKernelGGL(k_out_partial<8>, grid, dim3(kThreads), 0, s, a); break;
     case 16: hipLaunchKernelGGL(k_out_partial<16>, grid, dim3(kThreads), 0, s, a); break;

@@ -288,8 +288,9 @@ def triton_fused_sparse_mlp_decode_4bit(
 
     One row (a decode token) with the runtime's layouts (gate/up gathered
     [A*32, H], down gathered [H, A*32] with quant block 32) runs the fused
-    two-kernel decode path; anything else runs the composition of the
-    output/input linears, as the reference does."""
+    two-kernel decode path, several rows the output and input linears with
+    gate, up and act in one pass (the roundings of the composition); anything
+    else runs the composition, as the reference does."""
     device = require_device(x_flat, "x_flat")
     rows = int(x_flat.shape[0])
     H = int(gate_input_dim)
@@ -327,6 +328,33 @@ def triton_fused_sparse_mlp_decode_4bit(
             out.copy_(as_f16(down_bias, device).reshape(1, -1))
         else:
             out.zero_()
+        return out if x_flat.dtype != torch.bfloat16 else out.to(torch.bfloat16)
+    x = as_f16(x_flat, device)
+    rows_ok = (
+        bs == 32 and x.dim() == 2 and int(x.shape[1]) == H and active_idx.dim() == 2
+        and int(active_idx.shape[0]) == rows and int(active_idx.shape[1]) > 0 and flat_mask.dim() == 2
+        and int(flat_mask.shape[0]) == rows and rows > 0 and width > 0 and width % 32 == 0
+        and int(down_in_features) == width and int(up_input_dim) == H and int(down_out_features) > 0
+        and int(gate_quant_block_size) == int(up_quant_block_size)
+    )
+    if rows_ok:
+        gp, upk, dp = (_u8(t, device) for t in (gate_packed_weight, up_packed_weight, down_packed_weight))
+        rows_ok = (int(gp.numel()) == width * H // 2 and int(upk.numel()) == width * H // 2
+                   and int(dp.numel()) == int(down_out_features) * width // 2)
+    if rows_ok:
+        idx = _i32(active_idx, device)
+        kk, A = int(idx.shape[1]), width // 32
+        out = torch.empty((rows, int(down_out_features)), device=device, dtype=torch.float16)
+        ws = workspace(int(_lib.lib().nsmlp_fused_rows_workspace_bytes(rows, H, kk, A)), device)
+        _lib.call(
+            "nsmlp_fused_rows_gathered_f16",
+            ptr(x), rows, H, ptr(idx), kk, A, ptr(as_f16(flat_mask, device)),
+            ptr(gp), ptr(_f32(gate_absmax, device)), ptr(_f32(gate_code, device)), ptr(_opt_f16(gate_bias, device)),
+            ptr(upk), ptr(_f32(up_absmax, device)), ptr(_f32(up_code, device)), ptr(_opt_f16(up_bias, device)),
+            int(gate_quant_block_size),
+            ptr(dp), ptr(_f32(down_absmax, device)), ptr(_f32(down_code, device)), ptr(_opt_f16(down_bias, device)),
+            int(down_quant_block_size), int(down_out_features), ptr(out), ptr(ws), ws.numel(), stream_handle(device),
+        )
         return out if x_flat.dtype != torch.bfloat16 else out.to(torch.bfloat16)
     gate = triton_sparse_output_linear_4bit(
         x_flat, active_idx, flat_mask, packed_weight=gate_packed_weight, absmax=gate_absmax, code=gate_code,

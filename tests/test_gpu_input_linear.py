@@ -44,3 +44,50 @@ def test_input_linear_splits(gpu, orc, out, in_f, kk, bs, qbs, rows):
         mag = np.abs(prod).sum(axis=1) + np.abs(bias.astype(np.float64))
         bar = 2.0 ** -11 * np.abs(exact) + (kk * bs + 2) * 2.0 ** -23 * mag + 2.0 ** -24
         assert np.all(np.abs(y[r].astype(np.float64) - exact) <= bar), r
+
+
+@pytest.mark.parametrize("H,A,kk,rows,out,dtype", [
+    (256, 1, 1, 2, 32, torch.float16),
+    (512, 37, 9, 20, 512, torch.float16),   # entries left out, repeated and out of range
+    (1280, 20, 20, 3, 1280, torch.float16),
+    (2048, 16, 5, 4, 2048, torch.bfloat16),
+])
+def test_fused_rows_equal_composition(gpu, orc, H, A, kk, rows, out, dtype):
+    """The several-row fused call against its parts (output linears, silu
+    product, input linear), fp16 inputs bit for bit: masks that are not 0 or 1,
+    biases, entries of active_idx left out, repeated and out of range."""
+    from next_step_ai_amd import sparse_mlp as sm
+
+    print(f"fused rows H={H} A={A} kk={kk} rows={rows}", flush=True)
+    rng = np.random.default_rng(H + A)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+    half = lambda *s: t(rng.standard_normal(s).astype(np.float16))  # noqa: E731
+
+    def nf4(o, i, q):
+        p, a = orc.nf4_quantize((rng.standard_normal((o, i)) * 0.02).astype(np.float32), q)
+        return t(p), t(a)
+
+    (gp, ga), (up, ua), (dp, da) = nf4(A * 32, H, 64), nf4(A * 32, H, 64), nf4(out, A * 32, 32)
+    gb, ub, db = half(A * 32), half(A * 32), half(out)
+    code = torch.tensor(orc.nf4_code(), device=gpu)
+    idx = np.stack([rng.permutation(A)[:kk] for _ in range(rows)]).astype(np.int32)
+    if kk > 3:
+        idx[1, :3] = idx[1, 3], -1, A + 5
+    idx = t(idx)
+    mask = t((rng.integers(0, 4, (rows, A * 32)) / 2).astype(np.float16))
+    x = half(rows, H).to(dtype)
+    lin = dict(input_dim=H, quant_block_size=64, block_size=32, code=code)
+    g = sm.triton_sparse_output_linear_4bit(x.half(), idx, mask, packed_weight=gp, absmax=ga, bias=gb, **lin)
+    u = sm.triton_sparse_output_linear_4bit(x.half(), idx, mask, packed_weight=up, absmax=ua, bias=ub, **lin)
+    act = torch.empty_like(g)
+    from next_step_ai_amd import _lib
+    from next_step_ai_amd._runtime import ptr, stream_handle
+    _lib.call("nsmlp_silu_mul_f16", ptr(g), ptr(u), ptr(act), g.numel(), stream_handle(gpu))
+    ref = sm.triton_sparse_input_linear_4bit(act, idx, packed_weight=dp, absmax=da, code=code, out_features=out,
+                                             in_features=A * 32, quant_block_size=32, bias=db, block_size=32)
+    y = sm.triton_fused_sparse_mlp_decode_4bit(
+        x, idx, mask, gate_packed_weight=gp, gate_absmax=ga, gate_code=code, gate_input_dim=H,
+        gate_quant_block_size=64, gate_bias=gb, up_packed_weight=up, up_absmax=ua, up_code=code, up_input_dim=H,
+        up_quant_block_size=64, up_bias=ub, down_packed_weight=dp, down_absmax=da, down_code=code,
+        down_out_features=out, down_in_features=A * 32, down_quant_block_size=32, down_bias=db, block_size=32)
+    assert y.dtype == dtype and torch.equal(y, ref.to(dtype))
