@@ -33,7 +33,7 @@
 // Every sum is taken in a fixed order.
 //
 // At hidden 16384 and 8 tokens (1092 of 1664 blocks, 894 MB) gate/up takes 146
-// us (4.0 TB/s) and down 91 (3.2 TB/s): two waves a SIMD (the tokens'
+// us (4.0 TB/s) and down 87 (3.4 TB/s): two waves a SIMD (the tokens'
 // registers) leave the lookups' and MFMAs' latency partly open (without the
 // weight loads gate/up still takes 133 us); the loads are temporal, as a row's
 // 128-byte line serves two chunks (172 -> 158 us against nontemporal ones).
@@ -632,21 +632,12 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
     for (int c = 0; c < NCH; ++c) {
       Stage& su = st[c % PD];
       if (c < kc) {  // uniform over the wave
-#pragma unroll
-        for (int m = 0; m < RT; ++m) {
-          uint4 w = su.w[m];
-          swap16(w.x, w.y);
-          swap16(w.z, w.w);
-          swap32(w.x, w.z);
-          swap32(w.y, w.w);
-          const uint32_t dw[4] = {w.x, w.y, w.z, w.w};
-          float4_t cc[4][NT];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const half8_t bf = ft_codes8(dw[i], ad);
-#pragma unroll
-            for (int n = 0; n < NT; ++n) cc[i][n] = mfma16(x[c][i][n], bf, float4_t{0.0f, 0.0f, 0.0f, 0.0f});
-          }
+        // row tile m's lookups and MFMAs go out before the absmax multiplies
+        // m - 1's results: those lookups and MFMAs lie between an MFMA and the
+        // first read of its result (the last tile has the drain instead; with a
+        // drain a tile 91 us at hidden 16384, 8 tokens, now 87)
+        float4_t cc[2][4][NT];
+        auto scale = [&](int m) {
           // the lane's absmax, finite (a token that did not select the block
           // has a zero product with it), then every block's in all lane groups
           float a = su.am[m];
@@ -654,7 +645,6 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
           a = su.ok ? fminf(fmaxf(a, -3.0e38f), 3.0e38f) : 0.0f;
           float am[4];
           group_values(a, am);
-          mfma_drain();
           // |code sums| < 2^21 (32 products of |code| <= 1 and |act| < 2^16),
           // so a product outside the range needs an absmax of 4 or more
           if (__any(fabsf(a) >= 4.0f)) {
@@ -663,19 +653,39 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
 #pragma unroll
               for (int n = 0; n < NT; ++n)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) top = fmaxf(top, fabsf(cc[i][n][e] * am[i]));
+                for (int e = 0; e < 4; ++e) top = fmaxf(top, fabsf(cc[m & 1][i][n][e] * am[i]));
           }
 #pragma unroll
           for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int n = 0; n < NT; ++n)
 #pragma unroll
-              for (int e = 0; e < 4; ++e) acc[m][n][e] = __builtin_fmaf(cc[i][n][e], am[i], acc[m][n][e]);
+              for (int e = 0; e < 4; ++e) acc[m][n][e] = __builtin_fmaf(cc[m & 1][i][n][e], am[i], acc[m][n][e]);
           // summed here: left to itself the compiler moves the sums down to
           // their use and keeps (or spills) every product until then
 #pragma unroll
           for (int n = 0; n < NT; ++n) asm volatile("" : "+v"(acc[m][n]));
+        };
+#pragma unroll
+        for (int m = 0; m < RT; ++m) {
+          uint4 w = su.w[m];
+          swap16(w.x, w.y);
+          swap16(w.z, w.w);
+          swap32(w.x, w.z);
+          swap32(w.y, w.w);
+          const uint32_t dw[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const half8_t bf = ft_codes8(dw[i], ad);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) cc[m & 1][i][n] = mfma16(x[c][i][n], bf, float4_t{0.0f, 0.0f, 0.0f, 0.0f});
+          }
+          sched_fence();
+          if (m > 0) scale(m - 1);
+          sched_fence();
         }
+        mfma_drain();
+        scale(RT - 1);
       }
       issue(su, rg + (c + PD) / NCH, (c + PD) % NCH);
       sched_fence();
