@@ -19,8 +19,8 @@
 //              the end, zero for the tokens that did not select the block;
 //   k_ft_down  the same with K = the union's blocks: a wave holds the
 //              activations of its 4 NCH blocks and streams output rows past
-//              them; fp32 partial sums per group of waves;
-//   k_ft_fin   the partial sums in group order + bias, rounded once.
+//              them; partial sums per group of waves;
+//   k_ft_fin   the groups' partial sums + bias, rounded once.
 //
 // Weights go into the MFMAs as their fp16 code values (exact products, fp32
 // sums); the absmax multiplies the fp32 result of its own 64 columns
@@ -30,10 +30,14 @@
 // with v_permlane32_swap / v_permlane16_swap, 2 (4) VALU operations per 16
 // bytes, instead of narrower loads.
 //
-// Every sum is taken in a fixed order.
+// Gate/up sums are taken in a fixed order, which depends on the hidden size
+// and the number of token tiles only.  The down sums are exact: a block's place
+// in the union (its wave and group) depends on what the other tokens select,
+// and a token's output does not (see kFdGrid).
 //
 // At hidden 16384 and 8 tokens (1092 of 1664 blocks, 894 MB) gate/up takes 146
-// us (4.0 TB/s) and down 87 (3.4 TB/s): two waves a SIMD (the tokens'
+// us (4.0 TB/s) and down 104 (2.9 TB/s; 89 with fp32 sums, at 32 tokens 211
+// against 162): two waves a SIMD (the tokens'
 // registers) leave the lookups' and MFMAs' latency partly open (without the
 // weight loads gate/up still takes 133 us); the loads are temporal, as a row's
 // 128-byte line serves two chunks (172 -> 158 us against nontemporal ones).
@@ -53,6 +57,7 @@ constexpr int kFtLutWords = kRepLutBytes / 4;
 constexpr float kFtRange = 8388608.0f;  // 2^23, the range of the grouped down's partial products
 
 typedef unsigned u32x2v_t __attribute__((ext_vector_type(2)));
+typedef double double2_t __attribute__((ext_vector_type(2)));
 
 // Exchanges lanes 32..63 of a with lanes 0..31 of b.
 __device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {
@@ -120,6 +125,19 @@ __host__ __device__ inline int ft_down_groups(int nu, int H, int wgs, int NT) {
 // ------------------------------------------------------------ union list --
 constexpr int kFtMaxNB = 4096;
 constexpr int kFtMaxTok = 32;
+
+// Down sums: fp64, over multiples of 2^-31 (the unit of the grouped kernels'
+// fixed-point sums).  A wave's sum starts at kFdGrid = 1.5 2^21, whose ulp is
+// 2^-31, so every fma rounds the exact product of a block's fp32 code sum and
+// its absmax to that grid and adds it without another error, as long as the sum
+// stays below 2^20; sums on the grid add exactly in any order.  A product that
+// is a tie would round by the sum's parity: the absmax's lowest fp64 bit is set
+// (a relative 2^-52), so that a tie takes a product of 2^20.  Sums of 2^20 and
+// more lose the order independence, not the result.
+constexpr double kFdGrid = 3145728.0;
+__device__ __forceinline__ double fd_absmax(float a) {
+  return __longlong_as_double(__double_as_longlong((double)a) | 1ll);
+}
 
 __global__ void __launch_bounds__(1024) k_ft_list(FewTokArgs p) {
   __shared__ uint32_t mask[kFtMaxNB];
@@ -506,8 +524,8 @@ struct FdGeo {
   static constexpr int RT = 4 / NT;                          // row tiles of 16 rows per unit
   static constexpr int PD = NT == 1 ? 2 : 3;                 // units in flight (8 or 6 loads)
   static constexpr int kC2Word = kFtLutWords, kRefWord = kC2Word + 256, kCombWord = kRefWord + kFtWaves * NCH * 4 * 2;
-  static constexpr size_t kLds = (size_t)(kCombWord + 2 * kFtWaves * RT * NT * 256) * 4;
-  static_assert(kLds <= 160 * 1024 && NCH % PD == 0, "geometry");
+  static constexpr size_t kLds = (size_t)(kCombWord + kFtWaves * RT * NT * 512) * 4;
+  static_assert(kLds <= 160 * 1024 && NCH % PD == 0 && kCombWord % 4 == 0 && RT * NT == 4, "geometry");
 };
 
 template <bool DQ, bool HOST, int NT>
@@ -517,7 +535,7 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
   extern __shared__ __attribute__((aligned(16))) uint32_t lds[];  // no static LDS: the table is at LDS address 0
   const DecodeArgs& d = p.d;
   float* c2 = reinterpret_cast<float*>(lds + G::kC2Word);
-  float4_t* comb = reinterpret_cast<float4_t*>(lds + G::kCombWord);
+  double2_t* comb = reinterpret_cast<double2_t*>(lds + G::kCombWord);
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 15, g = lane >> 4;
@@ -613,7 +631,7 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
       }
     }
   };
-  float* part = p.part + (size_t)cg * M * H;
+  double* part = p.part + (size_t)cg * M * H;
   Stage st[PD];
 #pragma unroll
   for (int i = 0; i < PD; ++i) issue(st[i], rg_lo + i / NCH, i % NCH);
@@ -623,20 +641,26 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
   for (int m = 0; m < 4; ++m) ad[m] = (uint32_t)lane * 4u;
   float top = 0.0f;  // largest product seen where one may leave the range; inf or nan sums
   for (int rg = rg_lo; rg < rg_hi; ++rg) {
-    float4_t acc[RT][NT];
+    double acc[RT][NT][4];
 #pragma unroll
     for (int m = 0; m < RT; ++m)
 #pragma unroll
-      for (int n = 0; n < NT; ++n) acc[m][n] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[m][n][e] = kFdGrid;
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
       Stage& su = st[c % PD];
       if (c < kc) {  // uniform over the wave
         // row tile m's lookups and MFMAs go out before the absmax multiplies
         // m - 1's results: those lookups and MFMAs lie between an MFMA and the
-        // first read of its result (the last tile has the drain instead; with a
-        // drain a tile 91 us at hidden 16384, 8 tokens, now 87)
-        float4_t cc[2][4][NT];
+        // first read of its result (the last tile has the drain instead; a drain
+        // a tile cost 4 of 91 us at hidden 16384, 8 tokens)
+        // (with host copies and two token tiles the registers do not hold two
+        // tiles' products: a drain a tile there)
+        constexpr bool kAhead = !(HOST && NT == 2);
+        float4_t cc[kAhead ? 2 : 1][4][NT];  // tile m's: cc[m & kPar]
+        constexpr int kPar = kAhead ? 1 : 0;
         auto scale = [&](int m) {
           // the lane's absmax, finite (a token that did not select the block
           // has a zero product with it), then every block's in all lane groups
@@ -653,18 +677,22 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
 #pragma unroll
               for (int n = 0; n < NT; ++n)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) top = fmaxf(top, fabsf(cc[m & 1][i][n][e] * am[i]));
+                for (int e = 0; e < 4; ++e) top = fmaxf(top, fabsf(cc[m & kPar][i][n][e] * am[i]));
           }
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
+          for (int i = 0; i < 4; ++i) {
+            const double a64 = fd_absmax(am[i]);
 #pragma unroll
             for (int n = 0; n < NT; ++n)
 #pragma unroll
-              for (int e = 0; e < 4; ++e) acc[m][n][e] = __builtin_fmaf(cc[m & 1][i][n][e], am[i], acc[m][n][e]);
+              for (int e = 0; e < 4; ++e) acc[m][n][e] = __builtin_fma((double)cc[m & kPar][i][n][e], a64, acc[m][n][e]);
+          }
           // summed here: left to itself the compiler moves the sums down to
           // their use and keeps (or spills) every product until then
 #pragma unroll
-          for (int n = 0; n < NT; ++n) asm volatile("" : "+v"(acc[m][n]));
+          for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(acc[m][n][e]));
         };
 #pragma unroll
         for (int m = 0; m < RT; ++m) {
@@ -678,41 +706,48 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
           for (int i = 0; i < 4; ++i) {
             const half8_t bf = ft_codes8(dw[i], ad);
 #pragma unroll
-            for (int n = 0; n < NT; ++n) cc[m & 1][i][n] = mfma16(x[c][i][n], bf, float4_t{0.0f, 0.0f, 0.0f, 0.0f});
+            for (int n = 0; n < NT; ++n) cc[m & kPar][i][n] = mfma16(x[c][i][n], bf, float4_t{0.0f, 0.0f, 0.0f, 0.0f});
           }
-          sched_fence();
-          if (m > 0) scale(m - 1);
-          sched_fence();
+          if constexpr (kAhead) {
+            sched_fence();
+            if (m > 0) scale(m - 1);
+            sched_fence();
+          } else {
+            mfma_drain();
+            scale(m);
+          }
         }
-        mfma_drain();
-        scale(RT - 1);
+        if constexpr (kAhead) {
+          mfma_drain();
+          scale(RT - 1);
+        }
       }
       issue(su, rg + (c + PD) / NCH, (c + PD) % NCH);
       sched_fence();
     }
-    const int par = (rg - rg_lo) & 1;
+    if (rg > rg_lo) lds_barrier();  // the sums of the unit before have been read
 #pragma unroll
     for (int m = 0; m < RT; ++m)
 #pragma unroll
-      for (int n = 0; n < NT; ++n) {
+      for (int n = 0; n < NT; ++n)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) top = fabsf(acc[m][n][e]) < 3.4e38f ? top : kFtRange;
-        comb[((par * kFtWaves + wave) * 4 + m * NT + n) * 64 + lane] = acc[m][n];
-      }
+        for (int h = 0; h < 2; ++h) {
+          const double2_t v = {acc[m][n][2 * h] - kFdGrid, acc[m][n][2 * h + 1] - kFdGrid};
+          top = fabs(v[0]) < 1.0e300 && fabs(v[1]) < 1.0e300 ? top : kFtRange;
+          comb[((wave * 4 + m * NT + n) * 2 + h) * 64 + lane] = v;
+        }
     lds_barrier();
-    // four (row tile, token tile) sums of the 8 waves, by four waves
-    const int job = (wave - 4 * par) & 7;
-    if (job < 4) {
-      const int n = job % NT, m = job / NT;
-      float4_t y = comb[((par * kFtWaves) * 4 + job) * 64 + lane];
+    // four (row tile, token tile) sums of the 8 waves: two waves a tile, each
+    // two of a lane's four tokens
+    const int job = wave >> 1, h = wave & 1, n = job % NT, m = job / NT;
+    double2_t y = comb[(job * 2 + h) * 64 + lane];
 #pragma unroll
-      for (int w = 1; w < kFtWaves; ++w) y += comb[((par * kFtWaves + w) * 4 + job) * 64 + lane];
-      const int o = (rg * RT + m) * 16 + j;
+    for (int w = 1; w < kFtWaves; ++w) y += comb[((w * 4 + job) * 2 + h) * 64 + lane];
+    const int o = (rg * RT + m) * 16 + j;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = 16 * n + 4 * g + e;
-        if (t < M) part[(uint32_t)t * (uint32_t)H + (uint32_t)o] = y[e];
-      }
+    for (int e = 0; e < 2; ++e) {
+      const int t = 16 * n + 4 * g + 2 * h + e;
+      if (t < M) part[(uint32_t)t * (uint32_t)H + (uint32_t)o] = y[e];
     }
   }
   if (p.report_range && top >= kFtRange) atomicOr(d.status, NSMLP_STATUS_FIXED_RANGE);
@@ -723,8 +758,10 @@ __global__ void __launch_bounds__(256) k_ft_fin(FewTokArgs p) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
   const int CG = p.nu[1];
-  float y = 0.0f;
-  for (int s = 0; s < CG; ++s) y += p.part[(long long)s * n + i];
+  double sum = 0.0;
+#pragma unroll 4
+  for (int s = 0; s < CG; ++s) sum += p.part[(long long)s * n + i];
+  float y = (float)sum;
   if (p.d.down_bias != nullptr) y += h2f(p.d.down_bias[(int)(i % p.d.H)]);
   p.out[i] = f2h(y);
 }
@@ -806,15 +843,17 @@ size_t few_tokens_workspace(int H, int NB, int M, int k) {
   auto up = [](size_t v) { return (v + 255) / 256 * 256; };
   const long long nu = (long long)M * k < NB ? (long long)M * k : NB;
   const int cg = ft_groups_min((int)nu, ft_token_tiles(M)) + kFtGroupsTried - 1;
-  return 256 + 2 * up((size_t)NB * 4) + up((size_t)M * NB * 64) + up((size_t)cg * M * H * 4);
+  return 256 + 2 * up((size_t)NB * 4) + up((size_t)M * NB * 64) + up((size_t)cg * M * H * 8);
 }
 
 // Up to 32 tokens (two 16-token tiles of 128 VGPRs between them).  The grouped
 // kernels these replace there read the weights once per block as well, but
 // work tile by tile on token lists (hidden 16384, 1664 blocks, top-k 208,
-// double-quantised, whole prefill call with its route): 2 tokens 376 -> 132
-// us, 8 tokens 579 -> 290, 16 tokens 520 -> 367, 32 tokens 539 -> 473; hidden
-// 4096, 448 blocks, top-k 64: 8 tokens 144 -> 74, 24 tokens 103 -> 94.  Four
+// double-quantised, whole prefill call with its route, which is 6 us shorter
+// in the second figures): 2 tokens 366 -> 113 us, 8 tokens 578 -> 271, 16 tokens
+// 521 -> 342, 32 tokens 541 -> 505; hidden 4096, 448 blocks, top-k 64: 8 tokens
+// 144 -> 69, 32 tokens 103 -> 93; hidden 5120, 432 blocks, top-k 61, 32 tokens,
+// the closest: 109 -> 107 (its 40 chunks leave column waves idle).  Four
 // tiles (33 to 64 tokens, 2 chunks a wave) were slower than the grouped
 // kernels: 1138 against 544 and 167 against 106 us.
 bool few_tokens_shape(int H, int NB, int M) { return M <= kFtMaxTok && NB <= kFtMaxNB && H % 256 == 0; }
@@ -842,7 +881,7 @@ void launch_few_tokens(const FewTokArgs& args, void* ws, hipStream_t s) {
   w += up((size_t)d.NB * 4);
   p.act = (uint16_t*)w;
   w += up((size_t)p.M * d.NB * 64);
-  p.part = (float*)w;
+  p.part = (double*)w;
   const int gu = ft_columns(d.H, NT, &p.gu_cw, &p.gu_cgs);
   const long long n2 = (((long long)d.H * d.NB * 32 / d.qbs) + (1LL << d.dq_shift) - 1) >> d.dq_shift;
   p.gu_a2bytes = p.dn_a2bytes = (int)(n2 * 4);

@@ -805,7 +805,7 @@ struct FewTokArgs {
   int32_t* ublk;          // [NB] their ids, ascending
   uint32_t* umask;        // [NB] their tokens
   uint16_t* act;          // [M][NB 32] fp16, columns in union order
-  float* part;            // [groups][M][H] fp32
+  double* part;           // [groups][M][H] fp64, multiples of 2^-31
   int gu_cw, gu_cgs;      // gate/up column waves of a workgroup, column groups
   int gu_a2bytes, dn_a2bytes;
   // the rows of one dense matrix

@@ -103,3 +103,65 @@ def test_few_tokens_do_not_mix(gpu):
     others = [r for r in range(M) if r != 4]
     assert torch.equal(out2[others], out[others])
     assert not torch.isfinite(out2[4].float()).all()
+
+
+def _swap_selections(rng, NB, M, k, first):
+    """M ascending selections of k blocks, row 0 = first."""
+    sel = np.stack([np.sort(rng.permutation(NB)[:k]) for _ in range(M)]).astype(np.int32)
+    sel[0] = first
+    return sel
+
+
+@pytest.mark.parametrize("H,NB,k,Ms", [
+    (1024, 128, 6, (1, 5, 16)),        # M k < 2 NB: one and several groups of blocks
+    (4096, 448, 64, (1, 2, 13, 16)),   # on both sides of 2 NB
+    (2048, 96, 20, (17, 32)),          # two token tiles
+])
+def test_few_tokens_independent_of_other_selections(gpu, H, NB, k, Ms):
+    """A token's output bits do not depend on what the other tokens select,
+    nor (within a token tile) on how many there are: the down sums are exact,
+    so a block's place in the union does not matter."""
+    from next_step_ai_amd.synth import make_synthetic_layer, synth_normal_f16
+
+    print(f"few tokens, selections H={H} NB={NB} k={k}", flush=True)
+    L = make_synthetic_layer(H=H, I=32 * NB, R=16, seed=H + k, device=gpu, double_quant=True)
+    t = L.slot_table()
+    x = synth_normal_f16(31, (max(Ms), H), 1.0, gpu)
+    rng = np.random.default_rng(k)
+    first = np.sort(rng.permutation(NB)[:k]).astype(np.int32)
+    seen = []
+    for M in Ms:
+        for _ in range(3):
+            sel = torch.from_numpy(_swap_selections(rng, NB, M, k, first)).to(gpu)
+            seen.append(t.prefill(x[:M], sel, check=True)[0])
+    assert all(torch.equal(s, seen[0]) for s in seen), [int((s != seen[0]).sum()) for s in seen]
+
+
+@pytest.mark.parametrize("M,k", [(3, 10), (20, 10)])
+def test_few_tokens_down_sums_are_exact(gpu, M, k):
+    """Two blocks whose contributions cancel (the same weights, the down absmax
+    of one negated, about 2^15 each) leave the bits of the call without them:
+    the sums hold 2^-31 below 2^20, where fp32 sums would hold 2^-9."""
+    from next_step_ai_amd.synth import make_synthetic_layer, synth_normal_f16
+
+    H, NB = 1024, 64
+    L = make_synthetic_layer(H=H, I=32 * NB, R=16, seed=77, device=gpu)
+    t = L.slot_table(absmax="f32")
+    t.down_absmax[11] *= 65536.0
+    for name in ("gate_packed", "gate_absmax", "up_packed", "up_absmax", "down_packed"):
+        w = getattr(t, name)
+        w[40] = w[11]
+    t.down_absmax[40] = -t.down_absmax[11]
+    x = synth_normal_f16(78, (M, H), 1.0, gpu)
+    rng = np.random.default_rng(M)
+    others = np.setdiff1d(np.arange(NB), [11, 40])
+    pick = np.stack([rng.permutation(others)[: k - 2] for _ in range(M)])
+    without = np.sort(np.concatenate([pick, pick[:, :2]], axis=1), axis=1).astype(np.int32)  # repeats count once
+    both = np.sort(np.concatenate([pick, np.tile([11, 40], (M, 1))], axis=1), axis=1).astype(np.int32)
+    a = t.prefill(x, torch.from_numpy(without).to(gpu), check=True)
+    b = t.prefill(x, torch.from_numpy(both).to(gpu), check=True)
+    only = both.copy()
+    only[:, :] = 11
+    big = t.prefill(x, torch.from_numpy(only).to(gpu), check=True).float().abs().amax()
+    assert 2.0 ** 10 < float(big) < 2.0 ** 16, float(big)
+    assert torch.equal(a, b), int((a != b).sum())
