@@ -523,7 +523,8 @@ struct FdGeo {
   static constexpr int NCH = 6 / NT;                         // chunks a wave holds (96 VGPRs of activations)
   static constexpr int RT = 4 / NT;                          // row tiles of 16 rows per unit
   static constexpr int PD = NT == 1 ? 2 : 3;                 // units in flight (8 or 6 loads)
-  static constexpr int kC2Word = kFtLutWords, kRefWord = kC2Word + 256, kCombWord = kRefWord + kFtWaves * NCH * 4 * 2;
+  static constexpr int kC2Word = kFtLutWords, kRefWord = kC2Word + 256, kMaskWord = kRefWord + kFtWaves * NCH * 4 * 2,
+                       kNanWord = kMaskWord + kFtWaves * NCH * 4, kCombWord = kNanWord + 2 * RT * 16;
   static constexpr size_t kLds = (size_t)(kCombWord + kFtWaves * RT * NT * 512) * 4;
   static_assert(kLds <= 160 * 1024 && NCH % PD == 0 && kCombWord % 4 == 0 && RT * NT == 4, "geometry");
 };
@@ -556,18 +557,25 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
       if (tid < 256) c2[tid] = d.down.code2[tid];
     }
   }
+  // rows of a unit: the tokens whose sum is NaN (two units' buffers)
+  uint32_t* nans = lds + G::kNanWord;
+  if (tid < 2 * RT * 16) nans[tid] = 0;
   // (slot, or block id with bit 30 for a host copy; -1: none) and block id of
-  // the wave's blocks
+  // the wave's blocks, and the tokens that selected them
   int2* refs = reinterpret_cast<int2*>(lds + G::kRefWord) + wave * (NCH * 4);
+  uint32_t* masks = lds + G::kMaskWord + wave * (NCH * 4);
   if (lane < NCH * 4) {
     const int u = 4 * c_lo + lane;
     int2 e = make_int2(-1, 0);
+    uint32_t mask = 0;
     if (lane < 4 * kc && u < nu) {
+      mask = p.umask[u];
       const BlockRef br = resolve_id(d, p.ublk[u]);
       e.y = br.b;
       if (br.ok) e.x = br.dev ? (int)br.q : (0x40000000 | (int)br.q);
     }
     refs[lane] = e;
+    masks[lane] = mask;
   }
   half8_t x[NCH][4][NT];
   {
@@ -662,16 +670,24 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
         float4_t cc[kAhead ? 2 : 1][4][NT];  // tile m's: cc[m & kPar]
         constexpr int kPar = kAhead ? 1 : 0;
         auto scale = [&](int m) {
-          // the lane's absmax, finite (a token that did not select the block
-          // has a zero product with it), then every block's in all lane groups
+          // the lane's absmax, then every block's in all lane groups.  One
+          // that is not finite makes its row's sum NaN for the tokens that
+          // selected the block (weights 0 and infinite, or NaN), and only
+          // for those (the others' products with the block are zero).
           float a = su.am[m];
           if constexpr (DQ) a = dq_absmax(c2[su.qa[m]], a, d.down.offset);
-          a = su.ok ? fminf(fmaxf(a, -3.0e38f), 3.0e38f) : 0.0f;
+          a = su.ok ? a : 0.0f;
+          const bool wide = __any(!(fabsf(a) < 4.0f));
+          if (wide && !(fabsf(a) <= 3.402823466e38f)) {
+            atomicOr(&nans[((rg - rg_lo) & 1) * (RT * 16) + m * 16 + j], masks[c * 4 + g]);
+            top = kFtRange;
+            a = 0.0f;
+          }
           float am[4];
           group_values(a, am);
           // |code sums| < 2^21 (32 products of |code| <= 1 and |act| < 2^16),
           // so a product outside the range needs an absmax of 4 or more
-          if (__any(fabsf(a) >= 4.0f)) {
+          if (wide) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -725,7 +741,8 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
       issue(su, rg + (c + PD) / NCH, (c + PD) % NCH);
       sched_fence();
     }
-    if (rg > rg_lo) lds_barrier();  // the sums of the unit before have been read
+    if (rg > rg_lo) lds_barrier();  // the sums and marks of the unit before have been read
+    if (tid < RT * 16) nans[(~(rg - rg_lo) & 1) * (RT * 16) + tid] = 0;
 #pragma unroll
     for (int m = 0; m < RT; ++m)
 #pragma unroll
@@ -744,10 +761,11 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_down(FewTokArgs p) {
 #pragma unroll
     for (int w = 1; w < kFtWaves; ++w) y += comb[((w * 4 + job) * 2 + h) * 64 + lane];
     const int o = (rg * RT + m) * 16 + j;
+    const uint32_t nan = nans[((rg - rg_lo) & 1) * (RT * 16) + m * 16 + j];
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       const int t = 16 * n + 4 * g + 2 * h + e;
-      if (t < M) part[(uint32_t)t * (uint32_t)H + (uint32_t)o] = y[e];
+      if (t < M) part[(uint32_t)t * (uint32_t)H + (uint32_t)o] = (nan >> t) & 1u ? __builtin_nan("") : y[e];
     }
   }
   if (p.report_range && top >= kFtRange) atomicOr(d.status, NSMLP_STATUS_FIXED_RANGE);

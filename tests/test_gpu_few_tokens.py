@@ -165,3 +165,27 @@ def test_few_tokens_down_sums_are_exact(gpu, M, k):
     big = t.prefill(x, torch.from_numpy(only).to(gpu), check=True).float().abs().amax()
     assert 2.0 ** 10 < float(big) < 2.0 ** 16, float(big)
     assert torch.equal(a, b), int((a != b).sum())
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("M", [5, 20])
+def test_few_tokens_absmax_not_finite(gpu, M, bad):
+    """A down absmax that is NaN or infinite (its zero codes are then NaN
+    weights) makes the outputs of the tokens that selected its block NaN, and
+    leaves the others."""
+    from next_step_ai_amd.synth import make_synthetic_layer, synth_normal_f16
+
+    H, NB, k = 1024, 64, 8
+    L = make_synthetic_layer(H=H, I=32 * NB, R=16, seed=79, device=gpu)
+    t = L.slot_table(absmax="f32")
+    x = synth_normal_f16(80, (M, H), 1.0, gpu)
+    rng = np.random.default_rng(M)
+    sel = np.stack([np.sort(rng.permutation(NB - 1)[:k]) for _ in range(M)]).astype(np.int32)
+    sel[1::2, -1] = NB - 1
+    ids = torch.from_numpy(sel).to(gpu)
+    out = t.prefill(x, ids)
+    t.down_absmax[NB - 1, 3:] = bad
+    got = t.prefill(x, ids)
+    assert torch.equal(got[0::2], out[0::2]) and torch.equal(got[:, :3], out[:, :3])
+    hit = got[1::2, 3:].float()
+    assert torch.isnan(hit).all()
