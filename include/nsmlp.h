@@ -423,7 +423,11 @@ typedef struct nsmlp_nf4_matrix {
  * x [rows][in] fp16 (16-byte aligned), out [rows][out] fp16, out_f32
  * [rows][out] (nullable) the same sums before the fp16 rounding.  One pass
  * over the weight per row or two; with three rows or more, in a multiple of
- * 128 and qbs >= 64, per 32 rows.  in_features > 16384: use
+ * 128 and qbs >= 64, per 32 rows.  The two orders of fp32 sums differ: a row's
+ * bits are the same in every call of one or two rows, and the same in every
+ * call of three rows or more, but not across (fp32 rounding); a caller that
+ * compares the two bit for bit passes its rows one by one.
+ * Other shapes: the same bits in every call.  in_features > 16384: use
  * nsmlp_input_linear_nf4_f16 with every block active. */
 int nsmlp_dense_linear_nf4_f16(const nsmlp_nf4_matrix* w, const void* x, int rows, void* out, float* out_f32,
                                void* stream);

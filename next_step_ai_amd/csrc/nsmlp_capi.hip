@@ -1245,8 +1245,8 @@ int nsmlp_dense_linear_nf4_f16(const nsmlp_nf4_matrix* w, const void* x, int row
   }
   a.code = w->code;
   const int cus = device_cus();
+  const bool few = few_tokens_rows_fit(a, rows);
   for (int t = 0, nt; t < rows; t += nt) {
-    const bool few = few_tokens_rows_fit(a, rows - t);
     nt = rows - t >= 2 ? 2 : 1;
     if (!few && !plan_rows(a, nt, cus)) return set_error(NSMLP_EINVAL, "dense linear geometry not supported");
     a.x = (const uint16_t*)x + (long long)t * in;

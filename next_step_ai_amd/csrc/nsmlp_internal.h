@@ -879,7 +879,7 @@ struct RowsArgs {
 };
 bool plan_rows(RowsArgs& a, int nt, int cus);  // nt tokens per pass (1 or 2)
 void launch_rows(const RowsArgs& a, int nt, hipStream_t s);
-// Three rows or more: up to 32 a launch (returns how many).
+// Calls of three rows or more: up to 32 a launch (returns how many).
 bool few_tokens_rows_fit(const RowsArgs& a, int rows);
 int launch_few_tokens_rows(const RowsArgs& a, int rows, hipStream_t s);
 

@@ -71,7 +71,10 @@ def dense_linear_nf4(x: torch.Tensor, packed_weight: torch.Tensor, absmax: torch
                      *, out_f32: torch.Tensor | None = None) -> torch.Tensor:
     """``x [rows, in] @ W.T`` for a row-major NF4 ``W [out, in]`` (no bias),
     fp32 accumulation, fp16 result [rows, out].  ``out_f32`` ([rows, out]
-    fp32, optional) receives the sums before the fp16 rounding."""
+    fp32, optional) receives the sums before the fp16 rounding.  A row's bits
+    are the same in all calls of one or two rows, and in all calls of three or
+    more; between the two the order of the fp32 sums differs (``in`` a multiple
+    of 128 and ``quant_block_size`` >= 64; else all calls give the same)."""
     device = require_device(x, "x")
     xf = aligned16(as_f16(x, device).reshape(-1, int(in_features)))
     rows = int(xf.shape[0])

@@ -177,8 +177,8 @@ def test_dense_linear_tiny_and_ragged_shapes(gpu, orc, V, H, qbs, rows):
     (5, 128, 64, 3),          # part of one tile, one chunk
     (33, 256, 128, 16),       # a third tile of one row, a full token tile
     (1001, 4096, 64, 17),     # eight column waves, second token tile
-    (515, 5120, 64, 34),      # five chunks a wave; 32 rows, then a pass of two
-    (300, 10368, 128, 9),     # 81 chunks over two column groups, the last one part
+    (515, 5120, 64, 34),      # three column groups of four waves; 32 rows, then a pass of two
+    (300, 10368, 128, 9),     # 81 chunks over three column groups, the last one part
     (517, 16384, 256, 32),    # four column groups
     (131001, 128, 64, 20),    # two batches of tile sums a workgroup
 ])
@@ -209,3 +209,26 @@ def test_dense_linear_few_rows(gpu, orc, V, H, qbs, rows):
     out_i, _ = _run(gpu, x, pk, nested, code, V, H, qbs, with_f32=False)
     others = [r for r in range(rows) if r != 1]
     assert torch.equal(out_i[others], out_n[others]) and not torch.isfinite(out_i[1]).any()
+
+
+@pytest.mark.parametrize("V,H,qbs,first", [
+    (515, 4096, 64, 3),     # one column group of eight waves
+    (130, 5120, 64, 3),     # three of four waves
+    (67, 16384, 128, 3),    # four of eight waves
+    (37, 96, 32, 1),        # passes of one and two rows only
+])
+def test_dense_linear_row_independent_of_the_row_count(gpu, orc, V, H, qbs, first):
+    """A row's logits are the same bits in every call of `first` rows or more,
+    wherever the row stands and however many rows come with it."""
+    print(f"lm head row counts V={V} H={H}", flush=True)
+    rng = np.random.default_rng(V)
+    packed, absmax, x = _random_case(gpu, orc, rng, V, H, qbs, 34)
+    code = torch.tensor(orc.nf4_code(), device=gpu)
+    pk, am = torch.from_numpy(packed).to(gpu), torch.from_numpy(absmax).to(gpu)
+    ref, ref32 = _run(gpu, x, pk, am, code, V, H, qbs)
+    for rows in (1, 2, 3, 5, 8, 16, 17, 32, 33):
+        if rows < first:
+            continue
+        for at in (0, 34 - rows):
+            out, f32 = _run(gpu, x[at:at + rows], pk, am, code, V, H, qbs)
+            assert torch.equal(f32, ref32[at:at + rows]) and torch.equal(out, ref[at:at + rows]), (rows, at)
