@@ -74,6 +74,14 @@ def _opt_f16(t: torch.Tensor | None, device: torch.device) -> torch.Tensor | Non
     return None if t is None else as_f16(t.reshape(-1), device)
 
 
+def _projection(packed: torch.Tensor, absmax: torch.Tensor, code: torch.Tensor, bias: torch.Tensor | None,
+                device: torch.device) -> tuple[torch.Tensor | None, ...]:
+    """A projection's tensors as the kernels take them.  The caller holds the
+    tuple until the call is enqueued: a converted copy that nothing holds goes
+    back to the allocator, and the next copy takes its memory."""
+    return _u8(packed, device), _f32(absmax, device), _f32(code, device), _opt_f16(bias, device)
+
+
 def triton_sparse_mlp_decode_4bit_single_kernel_sm75(
     x_flat: torch.Tensor,
     active_blocks: torch.Tensor,
@@ -193,16 +201,15 @@ def triton_sparse_output_linear_4bit(
             raise RuntimeError("flat_mask width must be a multiple of block_size")
         A = width // int(block_size)
         mask = as_f16(flat_mask, device)
-        pw = _u8(packed_weight, device)
+        pw, am, cd, b16 = _projection(packed_weight, absmax, code, bias, device)
         if int(pw.numel()) != A * int(block_size) * int(input_dim) // 2:
             raise RuntimeError("packed_weight size does not match [A*block_size, input_dim] NF4 layout")
         nbytes = int(_lib.lib().nsmlp_output_linear_workspace_bytes(rows, kk, int(input_dim)))
         ws = workspace(nbytes, device)
         _lib.call(
             "nsmlp_output_linear_nf4_f16",
-            ptr(x), rows, int(input_dim), ptr(idx), kk, A, ptr(mask), ptr(pw), ptr(_f32(absmax, device)),
-            ptr(_f32(code, device)), int(quant_block_size), ptr(_opt_f16(bias, device)), int(block_size), ptr(out),
-            ptr(ws), ws.numel(), stream_handle(device),
+            ptr(x), rows, int(input_dim), ptr(idx), kk, A, ptr(mask), ptr(pw), ptr(am), ptr(cd),
+            int(quant_block_size), ptr(b16), int(block_size), ptr(out), ptr(ws), ws.numel(), stream_handle(device),
         )
     return out if out_dtype == torch.float16 else out.to(out_dtype)
 
@@ -246,14 +253,13 @@ def triton_sparse_input_linear_4bit(
         else:
             out.zero_()
     else:
-        pw = _u8(packed_weight, device)
+        pw, am, cd, b16 = _projection(packed_weight, absmax, code, bias, device)
         if int(pw.numel()) != int(out_features) * int(in_features) // 2:
             raise RuntimeError("packed_weight size does not match [out_features, in_features] NF4 layout")
         _lib.call(
             "nsmlp_input_linear_nf4_f16",
-            ptr(x), rows, int(in_features), ptr(idx), kk, ptr(pw), ptr(_f32(absmax, device)),
-            ptr(_f32(code, device)), int(quant_block_size), int(out_features), ptr(_opt_f16(bias, device)),
-            int(block_size), ptr(out), stream_handle(device),
+            ptr(x), rows, int(in_features), ptr(idx), kk, ptr(pw), ptr(am), ptr(cd), int(quant_block_size),
+            int(out_features), ptr(b16), int(block_size), ptr(out), stream_handle(device),
         )
     return out if out_dtype == torch.float16 else out.to(out_dtype)
 
@@ -308,8 +314,11 @@ def triton_fused_sparse_mlp_decode_4bit(
         x = aligned16(as_f16(x_flat, device).reshape(-1))
         idx = _i32(active_idx, device).reshape(-1)
         kk = int(idx.numel())
-        gp, upk, dp = (_u8(t, device) for t in (gate_packed_weight, up_packed_weight, down_packed_weight))
-        if int(gp.numel()) != width * H // 2 or int(upk.numel()) != width * H // 2 or int(dp.numel()) != H * width // 2:
+        gate = _projection(gate_packed_weight, gate_absmax, gate_code, gate_bias, device)
+        up = _projection(up_packed_weight, up_absmax, up_code, up_bias, device)
+        down = _projection(down_packed_weight, down_absmax, down_code, down_bias, device)
+        mask = as_f16(flat_mask, device)
+        if any(int(p[0].numel()) != width * H // 2 for p in (gate, up, down)):
             raise RuntimeError("packed weight sizes do not match the gathered [A*32, H] / [H, A*32] layouts")
         out = torch.empty((1, H), device=device, dtype=torch.float16)
         if kk > 0:
@@ -317,12 +326,8 @@ def triton_fused_sparse_mlp_decode_4bit(
             ws = workspace(nbytes, device)
             _lib.call(
                 "nsmlp_fused_decode_gathered_f16",
-                ptr(x), H, ptr(idx), kk, A, ptr(as_f16(flat_mask, device)),
-                ptr(gp), ptr(_f32(gate_absmax, device)), ptr(_f32(gate_code, device)), ptr(_opt_f16(gate_bias, device)),
-                ptr(upk), ptr(_f32(up_absmax, device)), ptr(_f32(up_code, device)), ptr(_opt_f16(up_bias, device)),
-                ptr(dp), ptr(_f32(down_absmax, device)), ptr(_f32(down_code, device)),
-                ptr(_opt_f16(down_bias, device)), int(gate_quant_block_size), ptr(out), ptr(ws), ws.numel(),
-                stream_handle(device),
+                ptr(x), H, ptr(idx), kk, A, ptr(mask), *map(ptr, gate), *map(ptr, up), *map(ptr, down),
+                int(gate_quant_block_size), ptr(out), ptr(ws), ws.numel(), stream_handle(device),
             )
         elif down_bias is not None:
             out.copy_(as_f16(down_bias, device).reshape(1, -1))
@@ -338,22 +343,22 @@ def triton_fused_sparse_mlp_decode_4bit(
         and int(gate_quant_block_size) == int(up_quant_block_size)
     )
     if rows_ok:
-        gp, upk, dp = (_u8(t, device) for t in (gate_packed_weight, up_packed_weight, down_packed_weight))
-        rows_ok = (int(gp.numel()) == width * H // 2 and int(upk.numel()) == width * H // 2
-                   and int(dp.numel()) == int(down_out_features) * width // 2)
+        rows_ok = (int(gate_packed_weight.numel()) == width * H // 2 and int(up_packed_weight.numel()) == width * H // 2
+                   and int(down_packed_weight.numel()) == int(down_out_features) * width // 2)
     if rows_ok:
         idx = _i32(active_idx, device)
+        gate = _projection(gate_packed_weight, gate_absmax, gate_code, gate_bias, device)
+        up = _projection(up_packed_weight, up_absmax, up_code, up_bias, device)
+        down = _projection(down_packed_weight, down_absmax, down_code, down_bias, device)
+        mask = as_f16(flat_mask, device)
         kk, A = int(idx.shape[1]), width // 32
         out = torch.empty((rows, int(down_out_features)), device=device, dtype=torch.float16)
         ws = workspace(int(_lib.lib().nsmlp_fused_rows_workspace_bytes(rows, H, kk, A)), device)
         _lib.call(
             "nsmlp_fused_rows_gathered_f16",
-            ptr(x), rows, H, ptr(idx), kk, A, ptr(as_f16(flat_mask, device)),
-            ptr(gp), ptr(_f32(gate_absmax, device)), ptr(_f32(gate_code, device)), ptr(_opt_f16(gate_bias, device)),
-            ptr(upk), ptr(_f32(up_absmax, device)), ptr(_f32(up_code, device)), ptr(_opt_f16(up_bias, device)),
-            int(gate_quant_block_size),
-            ptr(dp), ptr(_f32(down_absmax, device)), ptr(_f32(down_code, device)), ptr(_opt_f16(down_bias, device)),
-            int(down_quant_block_size), int(down_out_features), ptr(out), ptr(ws), ws.numel(), stream_handle(device),
+            ptr(x), rows, H, ptr(idx), kk, A, ptr(mask), *map(ptr, gate), *map(ptr, up), int(gate_quant_block_size),
+            *map(ptr, down), int(down_quant_block_size), int(down_out_features), ptr(out), ptr(ws), ws.numel(),
+            stream_handle(device),
         )
         return out if x_flat.dtype != torch.bfloat16 else out.to(torch.bfloat16)
     gate = triton_sparse_output_linear_4bit(

@@ -91,3 +91,48 @@ def test_fused_rows_equal_composition(gpu, orc, H, A, kk, rows, out, dtype):
         up_quant_block_size=64, up_bias=ub, down_packed_weight=dp, down_absmax=da, down_code=code,
         down_out_features=out, down_in_features=A * 32, down_quant_block_size=32, down_bias=db, block_size=32)
     assert y.dtype == dtype and torch.equal(y, ref.to(dtype))
+
+
+@pytest.mark.parametrize("rows", [1, 3])
+def test_converted_arguments_keep_their_values(gpu, orc, rows):
+    """Arguments of other types (bfloat16 masks and biases, float64 absmax and
+    codes) give what the same values of the kernels' types give: every converted
+    copy lives until the call is enqueued."""
+    from next_step_ai_amd import sparse_mlp as sm
+
+    print(f"converted arguments rows={rows}", flush=True)
+    H, A, kk = 512, 16, 6
+    rng = np.random.default_rng(rows)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+
+    def nf4(o, i, q):
+        p, a = orc.nf4_quantize((rng.standard_normal((o, i)) * 0.02).astype(np.float32), q)
+        return t(p), t(a)
+
+    (gp, ga), (up, ua), (dp, da) = nf4(A * 32, H, 64), nf4(A * 32, H, 64), nf4(H, A * 32, 32)
+    biases = [t(rng.standard_normal(n).astype(np.float32)).bfloat16() for n in (A * 32, A * 32, H)]
+    code = torch.tensor(orc.nf4_code(), device=gpu)
+    idx = t(np.stack([rng.permutation(A)[:kk] for _ in range(rows)]).astype(np.int32))
+    mask = t(rng.integers(0, 3, (rows, A * 32)).astype(np.float32) / 2).bfloat16()
+    x = t(rng.standard_normal((rows, H)).astype(np.float16))
+
+    def fused(half, wide):
+        return sm.triton_fused_sparse_mlp_decode_4bit(
+            x, idx, half(mask), gate_packed_weight=gp, gate_absmax=wide(ga), gate_code=wide(code), gate_input_dim=H,
+            gate_quant_block_size=64, gate_bias=half(biases[0]), up_packed_weight=up, up_absmax=wide(ua),
+            up_code=wide(code), up_input_dim=H, up_quant_block_size=64, up_bias=half(biases[1]),
+            down_packed_weight=dp, down_absmax=wide(da), down_code=wide(code), down_out_features=H,
+            down_in_features=A * 32, down_quant_block_size=32, down_bias=half(biases[2]), block_size=32)
+
+    def linears(half, wide):
+        g = sm.triton_sparse_output_linear_4bit(x, idx, half(mask), packed_weight=gp, absmax=wide(ga), code=wide(code),
+                                                input_dim=H, quant_block_size=64, bias=half(biases[0]), block_size=32)
+        y = sm.triton_sparse_input_linear_4bit(g, idx, packed_weight=dp, absmax=wide(da), code=wide(code),
+                                               out_features=H, in_features=A * 32, quant_block_size=32,
+                                               bias=half(biases[2]), block_size=32)
+        return torch.cat((g, y), dim=1)
+
+    for call in (fused, linears):
+        ref = call(lambda v: v.half(), lambda v: v)
+        assert torch.isfinite(ref.float()).all()
+        assert torch.equal(call(lambda v: v, lambda v: v.double()), ref), call.__name__
