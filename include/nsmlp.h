@@ -359,7 +359,7 @@ int nsmlp_fused_decode_gathered_f16(const void* x, int H, const int32_t* active_
  * and the input linear over act, with their roundings (fp16 gate, up and act).
  * x [rows][H], active_idx [rows][kk], flat_mask [rows][A*32], down packed
  * [out_features][A*32] NF4 with quant block down_qbs, out [rows][out_features].
- */
+ * Armed faults of its own name and of the three calls it replaces fire. */
 size_t nsmlp_fused_rows_workspace_bytes(int rows, int H, int kk, int A);
 int nsmlp_fused_rows_gathered_f16(const void* x, int rows, int H, const int32_t* active_idx, int kk, int A,
                                   const void* flat_mask, const uint8_t* gate_packed, const float* gate_absmax,

@@ -1069,6 +1069,37 @@ int nsmlp_fused_decode_gathered_f16(const void* x, int H, const int32_t* active_
   return run_decode(a, (hipStream_t)stream);
 }
 
+// The input linear's argument checks (nothing is launched before they pass).
+static int input_linear_args(LinearArgs& l, const void* x, int rows, int in_features, const int32_t* active_idx, int kk,
+                             const uint8_t* packed, const float* absmax, const float* code, int qbs, int out_features,
+                             const void* bias, int block_size, void* out) {
+  if (block_size <= 0 || block_size % 32 != 0)
+    return set_error(NSMLP_EINVAL, "block_size must be a multiple of 32 (got %d)", block_size);
+  if (rows <= 0 || kk <= 0 || out_features <= 0) return set_error(NSMLP_EINVAL, "rows, kk, out_features must be > 0");
+  if (in_features <= 0 || in_features % block_size != 0)
+    return set_error(NSMLP_EINVAL, "in_features %d must be a multiple of block_size %d", in_features, block_size);
+  if ((long long)kk * (block_size / 32) > INT32_MAX / 2) return set_error(NSMLP_EINVAL, "kk * block_size too large");
+  if (qbs <= 0 || qbs % 32 != 0 || in_features % qbs != 0)
+    return set_error(NSMLP_EINVAL, "quant block size %d must be a multiple of 32 dividing %d", qbs, in_features);
+  if (!x || !active_idx || !packed || !absmax || !code || !out) return set_error(NSMLP_EINVAL, "NULL tensor argument");
+  if (!aligned16(packed)) return set_error(NSMLP_EINVAL, "packed weight must be 16-byte aligned");
+  memset(&l, 0, sizeof(l));
+  l.x = (const uint16_t*)x;
+  l.rows = rows;
+  l.in_dim = in_features;
+  l.out_dim = out_features;
+  l.active_idx = active_idx;
+  l.kk = kk;
+  l.packed = packed;
+  l.absmax = absmax;
+  l.code = code;
+  l.qbs = qbs;
+  l.bias = (const uint16_t*)bias;
+  l.out = (uint16_t*)out;
+  l.bm = block_size / 32;
+  return NSMLP_OK;
+}
+
 size_t nsmlp_fused_rows_workspace_bytes(int rows, int H, int kk, int A) {
   return nsmlp_output_linear_workspace_bytes(rows, 2 * kk, H) + align_up((size_t)rows * A * 64);
 }
@@ -1080,8 +1111,11 @@ int nsmlp_fused_rows_gathered_f16(const void* x, int rows, int H, const int32_t*
                                   const uint8_t* down_packed, const float* down_absmax, const float* down_code,
                                   const void* down_bias, int down_qbs, int out_features, void* out, void* ws,
                                   size_t ws_bytes, void* stream) {
+  NSMLP_FAULT_POINT("fused_rows_gathered_f16");
+  // a fault of a part, which the call replaces, is the call's
   NSMLP_FAULT_POINT("output_linear_nf4_f16");
   NSMLP_FAULT_POINT("silu_mul_f16");
+  NSMLP_FAULT_POINT("input_linear_nf4_f16");
   if (rows <= 0 || kk <= 0 || A <= 0) return set_error(NSMLP_EINVAL, "rows, kk and A must be positive");
   if (H <= 0 || H % 256 != 0) return set_error(NSMLP_EINVAL, "input_dim %d must be a multiple of 256", H);
   if (qbs <= 0 || qbs % 32 != 0 || H % qbs != 0)
@@ -1093,7 +1127,11 @@ int nsmlp_fused_rows_gathered_f16(const void* x, int rows, int H, const int32_t*
   const size_t need = nsmlp_fused_rows_workspace_bytes(rows, H, kk, A);
   if (ws == nullptr || ws_bytes < need)
     return set_error(NSMLP_ENOSPC, "fused-rows workspace needs %zu bytes, got %zu", need, ws_bytes);
-  LinearArgs l;
+  uint16_t* act = (uint16_t*)((char*)ws + align_up(kCounterBytes));
+  LinearArgs l, down;
+  int rc = input_linear_args(down, act, rows, A * 32, active_idx, kk, down_packed, down_absmax, down_code, down_qbs,
+                             out_features, down_bias, 32, out);
+  if (rc) return rc;
   memset(&l, 0, sizeof(l));
   l.x = (const uint16_t*)x;
   l.rows = rows;
@@ -1113,14 +1151,13 @@ int nsmlp_fused_rows_gathered_f16(const void* x, int rows, int H, const int32_t*
   l.mask = (const uint16_t*)flat_mask;
   l.cs = choose_cs(H, rows * kk);
   l.splits = H / l.cs;
-  uint16_t* act = (uint16_t*)((char*)ws + align_up(kCounterBytes));
   l.out = act;
   l.part = (float*)((char*)act + align_up((size_t)rows * A * 64));
   launch_output_linear(l, (hipStream_t)stream);
-  const int rc = check_launch("fused rows gate/up");
+  rc = check_launch("fused rows gate/up");
   if (rc) return rc;
-  return nsmlp_input_linear_nf4_f16(act, rows, A * 32, active_idx, kk, down_packed, down_absmax, down_code, down_qbs,
-                                    out_features, down_bias, 32, out, stream);
+  launch_input_linear(down, (hipStream_t)stream);
+  return check_launch("fused rows down");
 }
 
 size_t nsmlp_output_linear_workspace_bytes(int rows, int kk, int in_dim) {
@@ -1169,31 +1206,10 @@ int nsmlp_input_linear_nf4_f16(const void* x, int rows, int in_features, const i
                                const uint8_t* packed, const float* absmax, const float* code, int qbs,
                                int out_features, const void* bias, int block_size, void* out, void* stream) {
   NSMLP_FAULT_POINT("input_linear_nf4_f16");
-  if (block_size <= 0 || block_size % 32 != 0)
-    return set_error(NSMLP_EINVAL, "block_size must be a multiple of 32 (got %d)", block_size);
-  if (rows <= 0 || kk <= 0 || out_features <= 0) return set_error(NSMLP_EINVAL, "rows, kk, out_features must be > 0");
-  if (in_features <= 0 || in_features % block_size != 0)
-    return set_error(NSMLP_EINVAL, "in_features %d must be a multiple of block_size %d", in_features, block_size);
-  if ((long long)kk * (block_size / 32) > INT32_MAX / 2) return set_error(NSMLP_EINVAL, "kk * block_size too large");
-  if (qbs <= 0 || qbs % 32 != 0 || in_features % qbs != 0)
-    return set_error(NSMLP_EINVAL, "quant block size %d must be a multiple of 32 dividing %d", qbs, in_features);
-  if (!x || !active_idx || !packed || !absmax || !code || !out) return set_error(NSMLP_EINVAL, "NULL tensor argument");
-  if (!aligned16(packed)) return set_error(NSMLP_EINVAL, "packed weight must be 16-byte aligned");
   LinearArgs l;
-  memset(&l, 0, sizeof(l));
-  l.x = (const uint16_t*)x;
-  l.rows = rows;
-  l.in_dim = in_features;
-  l.out_dim = out_features;
-  l.active_idx = active_idx;
-  l.kk = kk;
-  l.packed = packed;
-  l.absmax = absmax;
-  l.code = code;
-  l.qbs = qbs;
-  l.bias = (const uint16_t*)bias;
-  l.out = (uint16_t*)out;
-  l.bm = block_size / 32;
+  const int rc = input_linear_args(l, x, rows, in_features, active_idx, kk, packed, absmax, code, qbs, out_features, bias,
+                                   block_size, out);
+  if (rc) return rc;
   launch_input_linear(l, (hipStream_t)stream);
   return check_launch("input linear");
 }

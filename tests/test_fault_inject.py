@@ -129,3 +129,40 @@ def test_bad_environment_spec_fails_every_compute_call():
                                    "print(L.nsmlp_version())\n")
     lines = out.strip().splitlines()
     assert lines[0] == "-22" and "NSMLP_FAULT_INJECT" in lines[1] and int(lines[2]) >= 105
+
+
+def _fused_rows(lib, **over):
+    """nsmlp_fused_rows_gathered_f16 with plausible arguments (never read on
+    the host) and some of them replaced."""
+    p = 1 << 20
+    a = dict(x=p, rows=3, H=512, idx=p, kk=4, A=8, mask=p, gp=p, ga=p, gc=p, gb=None, up=p, ua=p, uc=p, ub=None, qbs=64,
+             dp=p, da=p, dc=p, db=None, down_qbs=32, out_features=512, out=p, ws=p, ws_bytes=1 << 30, stream=None)
+    a.update(over)
+    return lib.nsmlp_fused_rows_gathered_f16(*a.values())
+
+
+@pytest.mark.parametrize("name", ["fused_rows_gathered_f16", "output_linear_nf4_f16", "silu_mul_f16",
+                                  "input_linear_nf4_f16"])
+def test_fused_rows_fault_points(L, name):
+    """The several-row fused call fails by its own name and by those of the
+    calls it replaces, before anything is launched."""
+    from next_step_ai_amd import _lib
+
+    with _lib.injected_faults(f"{name}=nospc"):
+        assert _fused_rows(L) == -28
+        assert f"nsmlp_{name}".encode() in L.nsmlp_last_error()
+
+
+@pytest.mark.parametrize("over,text", [
+    (dict(down_qbs=48), b"quant block size 48"), (dict(out_features=0), b"out_features"),
+    (dict(dp=(1 << 20) + 8), b"16-byte aligned"), (dict(da=None), b"NULL"), (dict(qbs=96), b"quant block size 96"),
+    (dict(ws_bytes=64), b"workspace needs"),
+])
+def test_fused_rows_checks_every_argument_before_a_launch(L, over, text):
+    """Arguments of the down part too: an error of the launch itself (there is
+    no device here) would have another status."""
+    from next_step_ai_amd import _lib
+
+    _lib.fault_inject(None)
+    assert _fused_rows(L, **over) == (-28 if "ws_bytes" in over else -22)
+    assert text in L.nsmlp_last_error(), L.nsmlp_last_error()
