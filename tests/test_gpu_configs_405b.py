@@ -66,8 +66,8 @@ def test_partial_residency_405b(gpu, orc):
     assert st["decode_mlp_hot_blocks_hit"] == 2 * (K - MISSES) and st["decode_mlp_cold_blocks_streamed"] == 2 * MISSES
     print("[config 3] decode with 62 host misses bit-identical; 146 HBM + 62 host blocks counted", flush=True)
 
-    # prefill and dense guard through the same table (grouped down at 4
-    # tokens, the dense down over the scattered act at 16) and the all-resident one
+    # prefill (the few-token kernels, on both sides of M k = 2 NB) and dense
+    # guard through the same table and the all-resident one
     full_table = full.table
     xs = synth_normal_f16(sub_seed(3001, "x"), (16, H), 1.0, gpu)
     for M in (4, 16):

@@ -33,6 +33,8 @@ def _gather(orc, L, blocks):
     (9472, 1024, 9, 256),    # five splits, one item a round
     (14336, 1024, 32, 64),   # seven whole splits, every block
     (16128, 512, 5, 64),     # eight splits, the last 1792 columns
+    (1280, 67200, 9, 64),    # 2100 blocks: the selection takes eight scores a thread
+    (10240, 67584, 3, 128),  # the same over five splits
 ])
 def test_decode_hidden_sizes_match_oracle(gpu, orc, H, I, k, qbs):
     from next_step_ai_amd.synth import make_synthetic_layer
@@ -60,7 +62,10 @@ def test_decode_hidden_sizes_match_oracle(gpu, orc, H, I, k, qbs):
     (2048, 48, 48),
     (1280, 130, 97),
     (4096, 300, 300),   # tiles of a wave ending in 1 to 3 blocks
-    (16384, 520, 515),  # more blocks than one workgroup's activations hold at one group: the last tile is short
+    (8192, 300, 290),   # two block groups
+    (16384, 208, 203),  # one block group: the workgroup writes the output, a wave's last tile is short
+    (16384, 512, 512),  # the most blocks that one group's activations hold
+    (16384, 520, 515),  # more: the two-launch kernels, which read the row-major weight directly
 ])
 def test_gathered_down_equals_slot_path(gpu, orc, H, A, kk):
     """Row-major gathered blocks in any order, with entries left out (-1):
@@ -92,3 +97,40 @@ def test_gathered_down_equals_slot_path(gpu, orc, H, A, kk):
         holes[1::3] = -1
         kept = L.slot_table(resident_blocks=t(idx[[i for i in range(kk) if i % 3 != 1]]))
         assert torch.equal(fused(holes), kept.decode(L.x, t(idx)))
+
+
+@pytest.mark.parametrize("H,A,kk", [(256, 3, 2), (1280, 40, 33), (5120, 24, 17), (6144, 9, 9), (16384, 20, 13)])
+def test_gathered_biases_and_masks(gpu, orc, H, A, kk):
+    """Gate, up and down biases and a mask that is not 0 or 1 in the one-row
+    fused call, hidden sizes that fill their splits and that do not, against
+    float64: relL2 <= 1e-3 (fp16 activations and result)."""
+    from next_step_ai_amd.sparse_mlp import triton_fused_sparse_mlp_decode_4bit
+
+    print(f"biases and masks H={H} A={A} kk={kk}", flush=True)
+    rng = np.random.default_rng(H + A)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+
+    def nf4(o, i, q):
+        p, a = orc.nf4_quantize((rng.standard_normal((o, i)) * 0.02).astype(np.float32), q)
+        return t(p), t(a), orc.nf4_dequant(p, a, o * i, q).reshape(o, i).astype(np.float64)
+
+    (gp, ga, wg), (up, ua, wu), (dp, da, wd) = nf4(A * 32, H, 64), nf4(A * 32, H, 64), nf4(H, A * 32, 32)
+    gb, ub, db = (rng.standard_normal(n).astype(np.float16) for n in (A * 32, A * 32, H))
+    mask = (rng.integers(0, 4, (1, A * 32)) / 2).astype(np.float16)
+    x = rng.standard_normal((1, H)).astype(np.float16)
+    idx = np.sort(rng.permutation(A)[:kk]).astype(np.int32)
+    code = torch.tensor(orc.nf4_code(), device=gpu)
+    y = triton_fused_sparse_mlp_decode_4bit(
+        t(x), t(idx).reshape(1, -1), t(mask), gate_packed_weight=gp, gate_absmax=ga, gate_code=code, gate_input_dim=H,
+        gate_quant_block_size=64, gate_bias=t(gb), up_packed_weight=up, up_absmax=ua, up_code=code, up_input_dim=H,
+        up_quant_block_size=64, up_bias=t(ub), down_packed_weight=dp, down_absmax=da, down_code=code,
+        down_out_features=H, down_in_features=A * 32, down_quant_block_size=32, down_bias=t(db), block_size=32)
+    m = mask[0].astype(np.float64)
+    xd = x[0].astype(np.float64)
+    g, u = (wg @ xd + gb) * m, (wu @ xd + ub) * m
+    act = g / (1.0 + np.exp(-g)) * u
+    live = np.zeros(A * 32)
+    for b in idx:
+        live[b * 32:(b + 1) * 32] = 1.0
+    ref = wd @ (act * live) + db
+    assert orc.rel_l2(_np(y).reshape(-1).astype(np.float64), ref) <= 1e-3

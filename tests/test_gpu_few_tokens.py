@@ -44,6 +44,8 @@ def _check(orc, L, x, sel, out, what):
     (9216, 512, 16, 9, 64, True),      # 72 chunks: two column groups
     (16384, 1024, 32, 11, 256, False),  # two token tiles over four column groups
     (512, 32768, 32, 200, 64, True),   # 1024 blocks: several batches of tile sums a workgroup
+    (256, 131072, 32, 200, 64, False),  # 4096 blocks, the most: a union of about 3200
+    (256, 66560, 9, 700, 64, True),    # 2080 blocks: three a thread of the list, the last threads none
 ])
 def test_few_tokens_match_oracle(gpu, orc, H, I, M, k, qbs, dq):
     from next_step_ai_amd.synth import make_synthetic_layer, synth_normal_f16
@@ -189,3 +191,17 @@ def test_few_tokens_absmax_not_finite(gpu, M, bad):
     assert torch.equal(got[0::2], out[0::2]) and torch.equal(got[:, :3], out[:, :3])
     hit = got[1::2, 3:].float()
     assert torch.isnan(hit).all()
+
+
+def test_few_tokens_no_valid_block(gpu):
+    """A call whose every id is out of range: reported, zero outputs."""
+    from next_step_ai_amd.synth import make_synthetic_layer, synth_normal_f16
+
+    H, M, k = 512, 3, 2
+    L = make_synthetic_layer(H=H, I=1024, R=16, seed=12, device=gpu)
+    t = L.slot_table()
+    x = synth_normal_f16(13, (M, H), 1.0, gpu)
+    sel = torch.tensor([[-1, L.NB]] * M, dtype=torch.int32, device=gpu)
+    with pytest.raises(RuntimeError, match="out of range"):
+        t.prefill(x, sel, check=True)
+    assert not t.prefill(x, sel).any()

@@ -5,7 +5,9 @@ max(1e-3, e_ref) and relL2(gpu, fallback) <= 2 e_ref + 1e-3, where e_ref is
 the reference fallback restatement's own error (fp16 weights, gate, up, act).
 Double-quantised absmax must give bit-identical results to fp32 slots of the
 resolved absmax; repeated calls must be bit-identical (fixed-point sums in the
-grouped down, fixed-order fp32 sums in the dense down)."""
+grouped down, fixed-order fp32 sums in the dense down).  Calls of at most 32
+tokens run other kernels (quant blocks of 64 and more, at most 4096 blocks):
+tests/test_gpu_few_tokens.py."""
 import numpy as np
 import pytest
 import torch
@@ -48,7 +50,7 @@ def _check_rows(orc, y, ye, yf, rows, what):
 
 
 @pytest.mark.parametrize("H,I,M,k,seed", [
-    (2048, 8192, 4, 16, 3),        # M k < 2 NB: the grouped per-block down
+    (2048, 8192, 4, 16, 3),        # M k < 2 NB at few tokens (the few-token kernels)
     (1024, 4096, 40, 16, 1),       # one token group, few tokens per block (dense down over the scattered act)
     (4096, 14336, 256, 64, 2),     # 8B-shaped layer, M = 256 (two token groups)
     (2048, 8192, 300, 16, 5),      # dense down over a 256-token tile plus a 64-token tile
@@ -212,3 +214,54 @@ def test_prefill_quant_block_sizes(gpu, orc, qbs):
     sel_np = _np(sel).astype(np.int64)
     ye, yf = _oracle_rows(orc, L, x[rows], sel_np[rows])
     _check_rows(orc, _np(out_dq)[rows], ye, yf, range(len(rows)), f"prefill qbs={qbs}")
+
+
+@pytest.mark.parametrize("H,I,M,k,qbs", [
+    (2048, 16384, 40, 16, 64),    # 512 blocks, M k < 2 NB
+    (1024, 8192, 130, 3, 128),    # two token groups of 128
+    (2048, 8192, 4, 16, 32),      # few tokens, quant blocks of 32: not for the few-token kernels
+    (1024, 4160, 40, 30, 64),     # 130 blocks (not a multiple of 4), M k > 2 NB
+])
+def test_prefill_grouped_down(gpu, orc, H, I, M, k, qbs):
+    """The per-block down over fixed-point sums: rows against the oracle, the u8
+    absmax path and half of the blocks in host copies bit-identical, a token's
+    bits independent of what the others select."""
+    from next_step_ai_amd.synth import make_synthetic_layer, synth_normal_f16
+
+    print(f"grouped down H={H} I={I} M={M} k={k} qbs={qbs}", flush=True)
+    L = make_synthetic_layer(H=H, I=I, R=16, seed=H + M + k, device=gpu, qbs=qbs, double_quant=True)
+    x = synth_normal_f16(700 + M, (M, H), 1.0, gpu)
+    table = L.slot_table(absmax="dq")
+    sel = L.router().route(x, k)
+    out = table.prefill(x, sel, check=True)
+    assert torch.equal(out, table.prefill(x, sel)), "not deterministic"
+    assert torch.equal(out, L.slot_table(absmax="f32").prefill(x, sel))
+    half = torch.arange(0, L.NB, 2, dtype=torch.int32)
+    for absmax in ("dq", "f32"):
+        part = L.slot_table(resident_blocks=half, host_copy=True, absmax=absmax)
+        assert torch.equal(part.prefill(x, sel, check=True), out)
+    others = sel.roll(1, dims=0).clone()
+    others[0] = sel[0]
+    assert torch.equal(table.prefill(x, others)[0], out[0])
+    rows = sorted({0, 1, M // 2, M - 1})
+    sel_np = _np(sel).astype(np.int64)
+    for r in rows:
+        ye, yf = _oracle_rows(orc, L, x[r:r + 1], sel_np[r:r + 1])
+        _check_rows(orc, _np(out)[r:r + 1], ye, yf, [0], f"grouped down row {r}")
+
+
+@pytest.mark.parametrize("M", [33, 40])
+def test_prefill_grouped_down_reports_the_fixed_point_range(gpu, M):
+    """A partial of the grouped down past 2^23 raises in a checked call."""
+    from next_step_ai_amd.synth import make_synthetic_layer, synth_normal_f16
+
+    H, I, k = 1024, 16384, 8
+    L = make_synthetic_layer(H=H, I=I, R=16, seed=M, device=gpu)
+    t = L.slot_table(absmax="f32")
+    x = synth_normal_f16(M, (M, H), 1.0, gpu)
+    sel = L.router().route(x, k)
+    assert M * k < 2 * L.NB
+    t.prefill(x, sel, check=True)
+    t.down_absmax[int(sel[M - 1, 0])].fill_(1.0e8)
+    with pytest.raises(RuntimeError, match="fixed-point range"):
+        t.prefill(x, sel, check=True)

@@ -91,3 +91,20 @@ def test_noalloc_reports_unavailable_blocks_and_rejects_large_shapes(gpu):
     odd = make_synthetic_layer(H=1024, I=4096, R=16, seed=2105, device=gpu)
     with pytest.raises(RuntimeError, match="streaming kernels only"):
         _noalloc(odd.layer(16), odd.x)
+
+
+@pytest.mark.parametrize("H,I,k", [(6144, 2048, 33), (10240, 2048, 21), (12288, 1024, 32), (14336, 1024, 9)])
+def test_noalloc_splits_that_are_no_power_of_two(gpu, H, I, k):
+    """Hidden sizes of 3, 5, 6 and 7 splits of 2048 columns."""
+    from next_step_ai_amd.synth import make_synthetic_layer, synth_normal_f16
+
+    print(f"[noalloc] H={H}", flush=True)
+    layer = make_synthetic_layer(H=H, I=I, R=16, seed=H, device=gpu, double_quant=True).layer(k)
+    x = synth_normal_f16(H + 1, (H,), 1.0, gpu)
+    res = synth_normal_f16(H + 2, (H,), 1.0, gpu)
+    ref_out, ref_sel = layer.forward(x)
+    ref_add, _ = layer.forward(x, residual=res)
+    out, sel = _noalloc(layer, x)
+    out_add, _ = _noalloc(layer, x, residual=res)
+    torch.cuda.synchronize()
+    assert torch.equal(sel, ref_sel) and torch.equal(out, ref_out) and torch.equal(out_add, ref_add)
