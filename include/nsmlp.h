@@ -85,8 +85,11 @@ int nsmlp_fault_inject(const char* spec);
  *   NSMLP_STATUS_BLOCK_UNAVAILABLE: a selected block id was out of range, or
  *     not resident with no host copy (such a block contributed zero; the
  *     reference's gather raises there, RT:4530-4578);
- *   NSMLP_STATUS_FIXED_RANGE: a grouped prefill down partial was outside the
- *     fixed-point range (|v| >= 2^23, inf or nan); those outputs are wrong. */
+ *   NSMLP_STATUS_FIXED_RANGE: a prefill call with M k < 2 NB had a block's
+ *     down product outside the range of the fixed-point sums (|v| >= 2^23, inf
+ *     or nan).  Outputs of the grouped kernels are wrong there; those of up to
+ *     32 tokens are summed in fp64 and right where finite, and are reported
+ *     alike, so that a checked call does not depend on the token count. */
 #define NSMLP_STATUS_BLOCK_UNAVAILABLE 1
 #define NSMLP_STATUS_FIXED_RANGE 2
 int nsmlp_workspace_init(void* ws, size_t ws_bytes, void* stream);
@@ -265,12 +268,22 @@ int nsmlp_decode_layer_noalloc_f16(const nsmlp_router* router, const nsmlp_slot_
  *   out[t] = sum over b in sel[t] of Wd_b (silu(Wg_b x_t) * (Wu_b x_t))
  * x [M][H] fp16 (16-byte aligned), sel [M][k] int32 block ids (e.g. from
  * nsmlp_route_f16 with rows = M; an id repeated in a row counts once), out
- * [M][H] fp16.  Grouped per block on MFMA: fp16 operands (gate/up weights as
- * fp16(code * absmax), as the reference's dequant fallback rounds them,
- * RT:5439-5447; down weights as fp16 codes with the absmax applied to each
- * block's product in fp32), fp32 accumulation, act rounded to fp16 (RT:5459),
- * the down sums accumulated in fixed point (independent of scheduling).
- * M <= 65536 and M*H*2, M*k*64 < 2^31.  The workspace grows with M: when
+ * [M][H] fp16.  fp16 operands on MFMA, fp32 accumulation, act rounded to fp16
+ * (RT:5459).  Deterministic, and a token's output does not depend on what the
+ * other tokens select.  Two sets of kernels:
+ *   up to 32 tokens (quant blocks of 64 and more, at most 4096 blocks): one
+ *   pass over the union of the blocks.  Weights as fp16 codes, the absmax
+ *   applied to the fp32 sums of 64 columns (gate/up) or to a block's product
+ *   (down), the down sums in fp64 in units of 2^-31 (exact in any order below
+ *   2^20).  The order of the gate/up sums is one for calls of 1 to 16 tokens
+ *   and one for 17 to 32;
+ *   else grouped per block: gate/up weights as fp16(code * absmax), as the
+ *   reference's dequant fallback rounds them (RT:5439-5447); down weights as
+ *   fp16 codes with the absmax applied to each block's product in fp32, summed
+ *   in fixed point (units of 2^-31), or, with M k >= 2 NB, by the dense GEMM
+ *   in a fixed order of fp32 sums.
+ * M <= 65536 and M*H*2, M*k*64 < 2^31.  The workspace grows with M: past 32
+ * tokens, when
  * the tokens' blocks cover most of the layer (M k >= 2 NB) the down runs as
  * the dense GEMM over an act matrix [M][I] fp16 with S fp32 partials [M][H]
  * (at the 405B shape about 0.36 MB per token, 2.9 GB at 8192 tokens): run
@@ -356,7 +369,8 @@ int nsmlp_fused_decode_gathered_f16(const void* x, int H, const int32_t* active_
 
 /* The same call for several rows (version >= 106): the gate and up output
  * linears below in one pass, act = fp16(silu(gate) * up) at the active slots,
- * and the input linear over act, with their roundings (fp16 gate, up and act).
+ * and the input linear over act, with the roundings of those fp16 calls (fp16
+ * gate, up and act), bit for bit.
  * x [rows][H], active_idx [rows][kk], flat_mask [rows][A*32], down packed
  * [out_features][A*32] NF4 with quant block down_qbs, out [rows][out_features].
  * Armed faults of its own name and of the three calls it replaces fire. */

@@ -67,8 +67,8 @@ _STATUS_TEXT = {
         "a selected block id was out of range, or its block is neither in an HBM slot nor host-copied "
         "(it contributed zero to the output)",
     _lib.NSMLP_STATUS_FIXED_RANGE:
-        "a grouped prefill down partial was outside the fixed-point range (|v| >= 2^23, inf or nan); "
-        "those outputs are wrong",
+        "a prefill down product was outside the fixed-point range (|v| >= 2^23, inf or nan); those outputs are "
+        "wrong in a call of more than 32 tokens, and to be checked in a smaller one",
 }
 
 

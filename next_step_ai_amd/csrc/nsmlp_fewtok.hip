@@ -54,7 +54,10 @@ namespace {
 constexpr int kFtThreads = 512;
 constexpr int kFtWaves = 8;
 constexpr int kFtLutWords = kRepLutBytes / 4;
-constexpr float kFtRange = 8388608.0f;  // 2^23, the range of the grouped down's partial products
+// 2^23, the range of the grouped down's partial products: a product outside it
+// is right here, and reported where the grouped down would report it, so that a
+// checked call does not depend on the number of tokens
+constexpr float kFtRange = 8388608.0f;
 
 typedef unsigned u32x2v_t __attribute__((ext_vector_type(2)));
 typedef double double2_t __attribute__((ext_vector_type(2)));
@@ -837,10 +840,14 @@ void ft_launch(const FtKernel& k, int wgs, const FewTokArgs& p, hipStream_t s) {
 // The kernel (by the chunks a wave holds), column waves of a workgroup and
 // column groups (each a pass over the workgroup's tiles with its own tokens in
 // registers) for H columns: the fewest column groups, then the fewest chunk
-// slots, then the fewest chunks a wave (hidden 16384, 8 tokens: 8 chunks x 8
-// waves x 2 groups 146 us, 4 x 8 x 4 155, 6 x 8 x 3 177; hidden 4096, 12
-// tokens: 4 x 8 waves 23.1 us, 8 x 4 25.8; two token tiles at hidden 16384: 4
-// chunks 290 us, 3 chunks 350).
+// slots, then the fewest chunks a wave.  Whole prefill call, top-k an eighth of
+// the blocks, chunks x waves (groups where more than one), the rule's choice
+// first, in us.  8 tokens: hidden 3072 6x4 58, 4x8 58; 4096 4x8 63, 8x4 64; 5120
+// 5x8 72, 4x4(3) 76; 6144 6x8 79, 4x4(3) 82; 8192 8x8 98, 4x8(2) 100; 10240
+// 5x8(2) 132, 4x4(5) 131; 11264 6x8(2) 157, 4x8(3) 159; 12288 6x8(2) 167, 4x8(3)
+// 164; 14336 8x8(2) 216, 4x4(7) 217; 16384 8x8(2) 251, 4x8(4) 259.  24 tokens:
+// 3072 3x8 66, 4x8 69; 5120 3x8(2) 106, 4x4(3) 112; 6144 3x8(2) 111, 4x4(3) 118;
+// 7168 4x8(2) 138, 3x8(3) 147; 16384 4x8(4) 435, 3x8(6) 484.
 int ft_columns(int H, int NT, int* cw, int* cgs) {
   const int chunks = H / 128;
   int best = 0, cost = 0x7FFFFFFF;

@@ -356,7 +356,10 @@ __device__ __forceinline__ float16_t mfma32(half8_t a, half8_t b, float16_t c) {
 // compiler inserts: reads of a 16x16x32 result that follow its MFMA closely
 // have returned values that changed from run to run in the last elements
 // (written last), so MFMA results are read only after this drain (long
-// enough for the 32x32x16 shape's 16 passes too).
+// enough for the 32x32x16 shape's 16 passes too), or, in the few-token
+// kernels' pipelines, after at least the lookups (16 LDS reads, waited for, and
+// their address moves) and the MFMAs of the following tile or chunk, between
+// scheduling barriers; the last one of a loop has the drain.
 __device__ __forceinline__ void mfma_drain() {
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
@@ -798,7 +801,7 @@ struct FewTokArgs {
   const int32_t* sel;     // [M][k] block ids
   int k;
   uint16_t* out;          // [M][H] fp16
-  int report_range;       // report down products outside the fixed-point range
+  int report_range;       // report down products outside the grouped kernels' fixed-point range
   // set by launch_few_tokens: workspace and tiling
   int NT, wgs;            // 16-token tiles, workgroups of the products
   int32_t* nu;            // [2] union blocks, groups of the down's partial sums

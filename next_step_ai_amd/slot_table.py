@@ -339,10 +339,12 @@ class SparseMlpSlotTable:
     def prefill(self, x: torch.Tensor, sel: torch.Tensor, out: torch.Tensor | None = None, *,
                 check: bool = False) -> torch.Tensor:
         """M tokens ``x`` [M, H] with their own selected block ids ``sel``
-        [M, k] (the multi-token branch, RT:4857-4908 + RT:5453): grouped MFMA
-        gate/up/down over the union of the selected blocks; ``out`` [M, H] fp16.
-        ``check``: as in ``decode`` (also reports a grouped down partial
-        outside the fixed-point range)."""
+        [M, k] (the multi-token branch, RT:4857-4908 + RT:5453): MFMA gate/up/down
+        over the union of the selected blocks (one pass for up to 32 tokens,
+        grouped per block past that); ``out`` [M, H] fp16.  A token's output
+        does not depend on what the others select.  ``check``: as in ``decode``
+        (also reports, with M k < 2 NB, a down product outside the range of the
+        grouped kernels' fixed-point sums)."""
         x16 = x.reshape(-1, self.H).to(device=self.device, dtype=torch.float16).contiguous()
         s = sel.to(device=self.device, dtype=torch.int32).contiguous()
         M, k = int(x16.shape[0]), int(s.shape[-1])

@@ -295,8 +295,11 @@ def triton_fused_sparse_mlp_decode_4bit(
     One row (a decode token) with the runtime's layouts (gate/up gathered
     [A*32, H], down gathered [H, A*32] with quant block 32) runs the fused
     two-kernel decode path, several rows the output and input linears with
-    gate, up and act in one pass (the roundings of the composition); anything
-    else runs the composition, as the reference does."""
+    gate, up and act in one pass; anything else runs the composition, as the
+    reference does.  For fp16 tokens the several-row call gives the bits of the
+    composition; for bf16 tokens gate, up and act stay fp16 in it, where the
+    composition's calls hand them over in bf16 (so its result is the closer
+    one), and only the result is rounded to bf16."""
     device = require_device(x_flat, "x_flat")
     rows = int(x_flat.shape[0])
     H = int(gate_input_dim)

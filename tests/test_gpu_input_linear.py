@@ -136,3 +136,47 @@ def test_converted_arguments_keep_their_values(gpu, orc, rows):
         ref = call(lambda v: v.half(), lambda v: v)
         assert torch.isfinite(ref.float()).all()
         assert torch.equal(call(lambda v: v, lambda v: v.double()), ref), call.__name__
+
+
+def test_fused_rows_bf16_tokens(gpu, orc):
+    """bf16 tokens through the several-row call against float64: fp16 gate, up
+    and act (2^-11 each, 2 in the product) and a bf16 result, whose rounding has
+    an rms of 2^-9 / sqrt(3) of a value at most: relL2 <= 2e-3, and no further
+    off than the three calls it replaces, which hand over bf16."""
+    from next_step_ai_amd import sparse_mlp as sm
+
+    H, A, kk, rows = 2048, 16, 5, 4
+    rng = np.random.default_rng(77)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)  # noqa: E731
+
+    def nf4(o, i, q):
+        p, a = orc.nf4_quantize((rng.standard_normal((o, i)) * 0.02).astype(np.float32), q)
+        return t(p), t(a), orc.nf4_dequant(p, a, o * i, q).reshape(o, i).astype(np.float64)
+
+    (gp, ga, wg), (up, ua, wu), (dp, da, wd) = nf4(A * 32, H, 64), nf4(A * 32, H, 64), nf4(H, A * 32, 32)
+    code = torch.tensor(orc.nf4_code(), device=gpu)
+    idx = np.stack([rng.permutation(A)[:kk] for _ in range(rows)]).astype(np.int32)
+    mask = torch.ones((rows, A * 32), dtype=torch.float16, device=gpu)
+    x = t(rng.standard_normal((rows, H)).astype(np.float32)).bfloat16()
+    lin = dict(input_dim=H, quant_block_size=64, block_size=32, code=code, bias=None)
+    g = sm.triton_sparse_output_linear_4bit(x, t(idx), mask, packed_weight=gp, absmax=ga, **lin)
+    u = sm.triton_sparse_output_linear_4bit(x, t(idx), mask, packed_weight=up, absmax=ua, **lin)
+    assert g.dtype == torch.bfloat16
+    act = (torch.nn.functional.silu(g.float()) * u.float()).half().bfloat16()
+    parts = sm.triton_sparse_input_linear_4bit(act, t(idx), packed_weight=dp, absmax=da, code=code, out_features=H,
+                                               in_features=A * 32, quant_block_size=32, bias=None, block_size=32)
+    y = sm.triton_fused_sparse_mlp_decode_4bit(
+        x, t(idx), mask, gate_packed_weight=gp, gate_absmax=ga, gate_code=code, gate_input_dim=H,
+        gate_quant_block_size=64, gate_bias=None, up_packed_weight=up, up_absmax=ua, up_code=code, up_input_dim=H,
+        up_quant_block_size=64, up_bias=None, down_packed_weight=dp, down_absmax=da, down_code=code,
+        down_out_features=H, down_in_features=A * 32, down_quant_block_size=32, down_bias=None, block_size=32)
+    xd = x.float().cpu().numpy().astype(np.float64)
+    gd, ud = xd @ wg.T, xd @ wu.T
+    live = np.zeros((rows, A * 32))
+    for r in range(rows):
+        for b in idx[r]:
+            live[r, b * 32:(b + 1) * 32] = 1.0
+    ref = (gd / (1.0 + np.exp(-gd)) * ud * live) @ wd.T
+    err = [orc.rel_l2(v.float().cpu().numpy().astype(np.float64), ref) for v in (y, parts)]
+    print(f"bf16 rows: fused {err[0]:.2e}, parts {err[1]:.2e}", flush=True)
+    assert y.dtype == torch.bfloat16 and err[0] <= 2e-3 and err[0] <= err[1]
