@@ -36,7 +36,7 @@
 // and a token's output does not (see kFdGrid).
 //
 // At hidden 16384 and 8 tokens (1092 of 1664 blocks, 894 MB) gate/up takes 146
-// us (4.0 TB/s) and down 104 (2.9 TB/s; 89 with fp32 sums, at 32 tokens 211
+// us (4.0 TB/s) and down 107 (2.8 TB/s; 89 with fp32 sums, at 32 tokens 214
 // against 162): two waves a SIMD (the tokens'
 // registers) leave the lookups' and MFMAs' latency partly open (without the
 // weight loads gate/up still takes 133 us); the loads are temporal, as a row's
@@ -900,10 +900,11 @@ size_t few_tokens_workspace(int H, int NB, int M, int k) {
 // kernels these replace there read the weights once per block as well, but
 // work tile by tile on token lists (hidden 16384, 1664 blocks, top-k 208,
 // double-quantised, whole prefill call with its route, which is 6 us shorter
-// in the second figures): 2 tokens 366 -> 113 us, 8 tokens 578 -> 271, 16 tokens
-// 521 -> 342, 32 tokens 541 -> 505; hidden 4096, 448 blocks, top-k 64: 8 tokens
-// 144 -> 69, 32 tokens 103 -> 93; hidden 5120, 432 blocks, top-k 61, 32 tokens,
-// the closest: 109 -> 107 (its 40 chunks leave column waves idle).  Four
+// in the second figures): 2 tokens 366 -> 113 us, 8 tokens 578 -> 276, 16 tokens
+// 521 -> 345, 32 tokens 541 -> 513; hidden 4096, 448 blocks, top-k 64: 8 tokens
+// 144 -> 70, 32 tokens 103 -> 93; hidden 5120, 432 blocks, top-k 61, 32 tokens,
+// the closest: 109 -> 108 (its 40 chunks leave column waves idle; the grouped
+// kernels behind the present route would take about 103).  Four
 // tiles (33 to 64 tokens, 2 chunks a wave) were slower than the grouped
 // kernels: 1138 against 544 and 167 against 106 us.
 bool few_tokens_shape(int H, int NB, int M) { return M <= kFtMaxTok && NB <= kFtMaxNB && H % 256 == 0; }
