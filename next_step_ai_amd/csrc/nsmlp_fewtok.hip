@@ -293,13 +293,14 @@ __global__ void __launch_bounds__(kFtThreads, 2) k_ft_gu(FewTokArgs p) {
       const uint32_t f = ft_lane(tf, l);
       const bool ok = live && (int)f >= 0;
       const int chb = (icg * CW + cw) * NCH;
-      const int nr = !ok ? 0 : HEAD ? min(p.rows - 32 * pb - 16 * l, 16) : 16;  // the tile's rows
-      const rsrc_t rp = make_rsrc(reinterpret_cast<const void*>(ft_lane64(tw, l)), nr * (int)rs);
-      // temporal: a row's 128-byte line serves two chunks.  Columns past the
-      // last chunk read the next row (or zeros past the tile): their tokens
-      // are zero
-      const uint32_t voff = (uint32_t)j * rs + (uint32_t)(chb * 64) + 16u * (uint32_t)g;
       constexpr int c0 = U == 0 ? 0 : SU, c1 = U == 0 ? SU : NCH;
+      // the tile's rows; none for a unit past the last chunk where blocks may be
+      // host copies (hidden 5120, 32 tokens, half of them: 753 -> 729 us)
+      const int nr = !ok || (!HEAD && chb + c0 >= chunks) ? 0 : HEAD ? min(p.rows - 32 * pb - 16 * l, 16) : 16;
+      const rsrc_t rp = make_rsrc(reinterpret_cast<const void*>(ft_lane64(tw, l)), nr * (int)rs);
+      // temporal: a row's 128-byte line serves two chunks.  A unit's chunk past
+      // the last reads the next row (or zeros past the tile): its tokens are zero
+      const uint32_t voff = (uint32_t)j * rs + (uint32_t)(chb * 64) + 16u * (uint32_t)g;
 #pragma unroll
       for (int c = c0; c < c1; ++c) st.w[c - c0] = buf_ld16c(rp, voff + 64u * (uint32_t)c, 0);
       const rsrc_t ra = make_rsrc(reinterpret_cast<const void*>(ft_lane64(ta, l)), nr * (int)(A * (DQ ? 1u : 4u)));
