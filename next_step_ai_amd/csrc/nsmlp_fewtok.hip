@@ -809,10 +809,12 @@ constexpr FtKernel ft_down() {
    ft_gu<DQ, 1, 8, false>(), ft_gu<DQ, 2, 3, false>(), ft_gu<DQ, 2, 4, false>()}
 const FtKernel kFtGu[2][6] = {NSMLP_FT_GU(false), NSMLP_FT_GU(true)};
 #undef NSMLP_FT_GU
-// [dq][token tiles - 1]
-constexpr int kFtHeadChunks = 4;
-const FtKernel kFtHead[2][2] = {{ft_gu<false, 1, kFtHeadChunks, true>(), ft_gu<false, 2, kFtHeadChunks, true>()},
-                                {ft_gu<true, 1, kFtHeadChunks, true>(), ft_gu<true, 2, kFtHeadChunks, true>()}};
+// [dq][3 or 4 chunks][token tiles - 1]: the LM head has one order of its sums
+// for one and two token tiles, so a row's bits do not depend on the rows with it
+#define NSMLP_FT_HEAD(DQ) \
+  {{ft_gu<DQ, 1, 3, true>(), ft_gu<DQ, 2, 3, true>()}, {ft_gu<DQ, 1, 4, true>(), ft_gu<DQ, 2, 4, true>()}}
+const FtKernel kFtHead[2][2][2] = {NSMLP_FT_HEAD(false), NSMLP_FT_HEAD(true)};
+#undef NSMLP_FT_HEAD
 constexpr int kFtGuChunks[6] = {4, 5, 6, 8, 3, 4};
 // [dq][host copies][token tiles - 1]
 const FtKernel kFtDown[2][2][2] = {{{ft_down<false, false, 1>(), ft_down<false, false, 2>()},
@@ -828,7 +830,8 @@ void ft_set_lds() {
     };
     for (int q = 0; q < 2; ++q) {
       for (const FtKernel& k : kFtGu[q]) set(k);
-      for (const FtKernel& k : kFtHead[q]) set(k);
+      for (int c = 0; c < 2; ++c)
+        for (const FtKernel& k : kFtHead[q][c]) set(k);
       for (int h = 0; h < 2; ++h)
         for (const FtKernel& k : kFtDown[q][h]) set(k);
     }
@@ -864,28 +867,6 @@ int ft_columns(int H, int NT, int* cw, int* cgs) {
       }
     }
   return best;
-}
-
-// The same for the LM head, which has one order of its sums for one and two
-// token tiles (so a row's bits do not depend on the rows with it): always 4
-// chunks a wave; one group if 2 waves (or 1) hold the chunks, else the fewer
-// chunk slots of 4 and 8 waves, 8 of equals.  64000 rows, 8 and 24 tokens, in
-// us: hidden 4096 8 waves 34, 44, 4 waves 36, 49; hidden 6144 4 waves 50, 69, 8
-// waves (24 tokens) 77; hidden 8192 8 waves 67, 84, 4 waves 70, 94; hidden 12288
-// 8 waves 95, 120, 4 waves 101, 135.  Other chunk counts, 8 tokens: 8 chunks
-// 65 at hidden 8192 and 136 against 144 at 16384; 5 or 6 chunks 103 against 85
-// at 10240, 111 against 95 at 12288.
-void ft_head_columns(int H, int* cw, int* cgs) {
-  const int chunks = H / 128;
-  int best = 0x7FFFFFFF;
-  for (int w = kFtWaves; w >= 1; w /= 2) {
-    const int c = (chunks + w * kFtHeadChunks - 1) / (w * kFtHeadChunks);
-    if (c * w < best && (w >= 4 || c == 1)) {
-      best = c * w;
-      *cw = w;
-      *cgs = c;
-    }
-  }
 }
 
 }  // namespace
@@ -948,10 +929,13 @@ void launch_few_tokens(const FewTokArgs& args, void* ws, hipStream_t s) {
 // The few-row LM head against passes of one or two rows (k_rows_rep), fp32
 // absmax, 128256 rows, one call: hidden 4096, 3 rows 145 -> 62 us, 5 rows 227 ->
 // 62 (4.8 TB/s), 16 rows 701 -> 67, 32 rows 1397 -> 90; hidden 16384, 5 rows 831
-// -> 236.  Calls of one and two rows stay there: they give bit-equal logits with
+// -> 227.  Calls of one and two rows stay there: they give bit-equal logits with
 // each other, and one row is faster (190 us at hidden 16384, 51 at 4096).  A call
-// of three rows or more takes every row here, so that all of its rows, and the
-// rows of all such calls, have one order of sums.
+// of three rows or more takes every row here, and the column split is the
+// two-tile one for every number of rows, so that all the rows of all such calls
+// have one order of sums; 4 rows against the one-tile split: hidden 9216 189 ->
+// 151 us, 12288 205 -> 178, 5120 99 -> 98, 16384 230 -> 226, 2304 44 -> 47, the
+// worst.
 // MFMA chunks want whole 128 columns, and an absmax of whole 64-column halves.
 bool few_tokens_rows_fit(const RowsArgs& a, int rows) {
   return rows > 2 && a.in % 128 == 0 && a.qbs_shift >= 6 && device_cus() >= 64;
@@ -982,9 +966,9 @@ int launch_few_tokens_rows(const RowsArgs& a, int rows, hipStream_t s) {
   p.out_f32 = a.out_f32;
   p.gu_a2bytes = a.a2_bytes;
   p.NT = ft_token_tiles(p.M);
-  ft_head_columns(a.in, &p.gu_cw, &p.gu_cgs);
+  const int gu = ft_columns(a.in, 2, &p.gu_cw, &p.gu_cgs);  // the two-tile choice, whatever the rows
   ft_set_lds();
-  ft_launch(kFtHead[a.dq ? 1 : 0][p.NT - 1], device_cus(), p, s);
+  ft_launch(kFtHead[a.dq ? 1 : 0][kFtGuChunks[gu] - 3][p.NT - 1], device_cus(), p, s);
   return p.M;
 }
 

@@ -177,8 +177,9 @@ def test_dense_linear_tiny_and_ragged_shapes(gpu, orc, V, H, qbs, rows):
     (5, 128, 64, 3),          # part of one tile, one chunk
     (33, 256, 128, 16),       # a third tile of one row, a full token tile
     (1001, 4096, 64, 17),     # eight column waves, second token tile
-    (515, 5120, 64, 34),      # three column groups of four waves; 32 rows, then a pass of two
+    (515, 5120, 64, 34),      # two groups of eight waves of three chunks; 32 rows, then a pass of two
     (300, 10368, 128, 9),     # 81 chunks over three column groups, the last one part
+    (61, 9216, 64, 20),       # three groups of three chunks, all full
     (517, 16384, 256, 32),    # four column groups
     (131001, 128, 64, 20),    # two batches of tile sums a workgroup
 ])
@@ -213,8 +214,8 @@ def test_dense_linear_few_rows(gpu, orc, V, H, qbs, rows):
 
 @pytest.mark.parametrize("V,H,qbs,first", [
     (515, 4096, 64, 3),     # one column group of eight waves
-    (130, 5120, 64, 3),     # three of four waves
-    (67, 16384, 128, 3),    # four of eight waves
+    (130, 5120, 64, 3),     # two, of three chunks a wave
+    (67, 16384, 128, 3),    # four
     (37, 96, 32, 1),        # passes of one and two rows only
 ])
 def test_dense_linear_row_independent_of_the_row_count(gpu, orc, V, H, qbs, first):
